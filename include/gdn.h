@@ -296,10 +296,10 @@ typedef struct gdn_qlinear gdn_qlinear;
 
 /* Merge nparts MLX-format parts (device pointers, part i has part_rows[i]
  * output rows) into one layer with N = sum(part_rows) outputs and repack it
- * for the kernel on `device`. The layer owns its memory (about N*K/2 +
- * 3*N*K/32 bytes, plus K/512 * 64 * N f32 partial sums for layers whose
- * decode-sized calls split K: K > 2048, or N < 8192 with K >= 1024); the
- * sources are only read, and may be freed once this returns (it synchronises
+ * for the kernel on `device`. The layer owns its memory: about N*K/2 +
+ * 3*N*K/32 bytes; 16384 * 3*K/32 bytes for a call's group sums; and for layers
+ * whose calls can split K (K >= 1024 and N <= 16384, or K > 2048) f32 partial
+ * sums, 16 MiB or K/512 * 64 * N of them if that is more. The sources are only read, and may be freed once this returns (it synchronises
  * `stream`). Supported: bits 4, group_size 64, K a multiple of 512 up to
  * 4096, part_rows multiples of 16. */
 gdn_status gdn_qlinear_create(int32_t K, int32_t nparts, const int32_t* part_rows,

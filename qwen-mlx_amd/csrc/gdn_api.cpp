@@ -697,15 +697,12 @@ struct gdn_qlinear {
   uint16_t* bias = nullptr;  // [Npad, G] bf16
   uint16_t* nsc = nullptr;   // [Npad, G] bf16, -128 * scales
   float* part = nullptr;     // K-slice partials of decode-sized calls [slices][64][Npad] f32
+  uint16_t* xsum = nullptr;  // split group sums of a call's rows [kQLinearSumRows/64][3][64][G] bf16
 };
 
 static void qlinear_release(gdn_qlinear* q) {
   if (!q) return;
-  if (q->wp) (void)hipFree(q->wp);
-  if (q->sp) (void)hipFree(q->sp);
-  if (q->bias) (void)hipFree(q->bias);
-  if (q->nsc) (void)hipFree(q->nsc);
-  if (q->part) (void)hipFree(q->part);
+  if (q->wp) (void)hipFree(q->wp);  // one allocation holds all of the layer's arrays
   delete q;
 }
 
@@ -747,20 +744,30 @@ gdn_status gdn_qlinear_create(int32_t K, int32_t nparts, const int32_t* part_row
   q->device = device;
   const size_t wbytes = (size_t)q->Npad * K / 2, gbytes = (size_t)q->Npad * q->G * 2;
   const int slices = gdn::qlinear_decode_slices(K, q->Npad);
-  const size_t pbytes = slices > 1 ? (size_t)slices * 64 * q->Npad * sizeof(float) : 0;
-  if (hipMalloc(&q->wp, wbytes) != hipSuccess || hipMalloc(&q->sp, gbytes) != hipSuccess ||
-      hipMalloc(&q->bias, gbytes) != hipSuccess || hipMalloc(&q->nsc, gbytes) != hipSuccess ||
-      (pbytes && hipMalloc(&q->part, pbytes) != hipSuccess)) {
+  // partials of K slices: of decode-sized calls, and of tiles (K of at least two slices)
+  size_t pbytes = slices > 1 ? (size_t)slices * 64 * q->Npad * sizeof(float) : 0;
+  const size_t tbytes = (size_t)gdn::kQLinearPartTiles * 64 * 128 * sizeof(float);
+  if (K >= 1024 && 2 * (q->Npad / 128) * 2 <= gdn::kQLinearPartTiles && pbytes < tbytes) pbytes = tbytes;
+  const size_t xbytes = (size_t)gdn::kQLinearSumRows * 3 * q->G * 2;
+  // one allocation: weights, scales, biases, -128 scales (cleared: rows past N),
+  // then the workspaces; every size is a multiple of 256 (Npad of 128, G of 8)
+  const size_t cleared = wbytes + 3 * gbytes;
+  if (hipMalloc(&q->wp, cleared + pbytes + xbytes) != hipSuccess) {
+    (void)hipGetLastError();
+    q->wp = nullptr;
     qlinear_release(q);
     return fail(GDN_ERR_OOM, "gdn_qlinear_create: hipMalloc of %zu bytes failed",
-                wbytes + 3 * gbytes);
+                cleared + pbytes + xbytes);
   }
+  char* base = static_cast<char*>(q->wp);
+  q->sp = reinterpret_cast<uint16_t*>(base + wbytes);
+  q->bias = reinterpret_cast<uint16_t*>(base + wbytes + gbytes);
+  q->nsc = reinterpret_cast<uint16_t*>(base + wbytes + 2 * gbytes);
+  if (pbytes) q->part = reinterpret_cast<float*>(base + cleared);
+  q->xsum = reinterpret_cast<uint16_t*>(base + cleared + pbytes);
   hipStream_t s = as_stream(stream);
   hipError_t e;
-  if ((e = hipMemsetAsync(q->wp, 0, wbytes, s)) != hipSuccess ||
-      (e = hipMemsetAsync(q->sp, 0, gbytes, s)) != hipSuccess ||
-      (e = hipMemsetAsync(q->bias, 0, gbytes, s)) != hipSuccess ||
-      (e = hipMemsetAsync(q->nsc, 0, gbytes, s)) != hipSuccess) {
+  if ((e = hipMemsetAsync(q->wp, 0, cleared, s)) != hipSuccess) {
     qlinear_release(q);
     return hip_fail(e, "gdn_qlinear_create: clear");
   }
@@ -883,6 +890,7 @@ gdn_status qlinear_forward(const gdn_qlinear* q, const uint16_t* x, int64_t x_st
   a.part = q->part;
   a.defer = defer;
   a.xsplit = M <= 64 ? xsplit : nullptr;
+  a.xsum = q->xsum;
   a.stream = as_stream(stream);
   hipError_t e = gdn::launch_qlinear(a);
   if (e != hipSuccess) return hip_fail(e, "gdn_qlinear_forward launch");

@@ -252,8 +252,15 @@ struct QLinearArgs {
                       // partials here instead of writing y (nslice = 0 when y was written)
   const uint16_t* xsplit;  // or null: x's 64-column group sums as three bf16 parts
                            // [3][64][K/64] (launch_add_norm's), used by decode shapes
+  uint16_t* xsum;     // workspace of kQLinearSumRows rows' split sums (prefill shapes)
   hipStream_t stream;
 };
+// Rows whose split group sums a layer's workspace holds (a multiple of 64):
+// larger calls go in pieces of this many rows.
+constexpr int kQLinearSumRows = 16384;
+// 64 x 128 f32 tiles (32 KiB each) of a layer's partial-sum workspace: a
+// K-sliced call of M > 64 rows is at most this many work-groups.
+constexpr int kQLinearPartTiles = 512;
 
 hipError_t launch_qlinear_pack(const QLinearPackArgs& a);
 hipError_t launch_qlinear(const QLinearArgs& a);

@@ -31,7 +31,15 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kStageK = 128;    // k per pipeline stage: two groups
-constexpr int kMaxGroups = 64;  // K <= 4096
+// Calls of at least kSumTiles tiles (three rounds of the 768 work-groups that
+// fit the chip) on layers of at least kSumColumns columns form the group sums
+// once up front (qlinear_xsum_kernel) instead of in every column tile: 880 us
+// against 928 at 16384 x 2048 -> 12,352 and 199 against 215 at M = 3688. Fewer
+// tiles do not pay the extra launch (M = 300: 27.0 us against 25.3), nor does a
+// narrow layer, whose 16 column tiles share a row's sums (K = 4096 -> 2048:
+// 319 us against 309 at M = 16,384).
+constexpr int kSumTiles = 2304;
+constexpr int kSumColumns = 4096;
 constexpr int kWideDecodeN = 131072;  // decode-sized calls at least this wide use 64 x 128 tiles
 
 __device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
@@ -110,294 +118,189 @@ __global__ void qlinear_pack_kernel(const uint32_t* __restrict__ w, const uint16
   }
 }
 
-// y[m, n] for a work-group tile of MT = 16*MW*WM rows (m) by NT = 16*NW*WN
-// columns (n); wave (wm, wn) owns MW row fragments and NW column fragments.
-// The weight fragment is the MFMA A operand (16 n x 32 k), the activation
-// fragment the B operand (32 k x 16 m), so each lane ends with four
-// consecutive n of one row m: D[4c + r][m], c = lane/16.
-// x is staged through LDS in stages of 128 k (double buffered, rows of 256 B
-// with the 16-byte chunk index XOR-swizzled by row so fragment reads are
-// conflict-free); weights and scales go straight from global memory to
-// registers one stage ahead.
-template <int MW, int NW, int WM, int WN>
-__global__ __launch_bounds__(256) void qlinear_kernel(
-    const uint16_t* __restrict__ x, int64_t xs, int M, int K, const u32x4* __restrict__ wp,
-    const uint16_t* __restrict__ sp, const uint16_t* __restrict__ bias,
-    const uint16_t* __restrict__ nsc, int N, uint16_t* __restrict__ y, int64_t ys) {
-  static_assert(WM * WN == 4, "four waves per work-group");
-  constexpr int MT = 16 * MW * WM, NT = 16 * NW * WN;
-  constexpr int XROW = kStageK * 2;  // bytes per staged x row
-  constexpr int SJ = MT / 16;        // staged uint4 per thread per stage
-  __shared__ __align__(16) uint8_t xl[2][MT * XROW];
-  __shared__ float sx[kMaxGroups * MT];  // X_g[m] at sx[g*MT + m]
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / WN, wn = wave % WN;
-  const int G = K >> 6, P = K >> 7;
-  const int m0 = blockIdx.y * MT;
-  const int f0 = blockIdx.x * (NT / 16) + wn * NW;  // first column fragment of the wave
-  const int r16 = lane & 15, c4 = lane >> 4;
-
-  // staging: thread -> rows srow + 16j, 16-byte chunk sch
-  const int srow = tid >> 4, sch = tid & 15;
-  const int sdst = srow * XROW + ((sch ^ (srow & 15)) << 4);
-  const uint16_t* xsrc[SJ];
-#pragma unroll
-  for (int j = 0; j < SJ; ++j) {
-    const int r = min(m0 + srow + 16 * j, M - 1);
-    xsrc[j] = x + (int64_t)r * xs + sch * 8;
-  }
-  u32x4 stg[SJ];
-  const u32x4* wsrc[NW];
-  const u32x4* ssrc[NW];
-#pragma unroll
-  for (int i = 0; i < NW; ++i) {
-    wsrc[i] = wp + (int64_t)(f0 + i) * P * 64 + lane;
-    ssrc[i] = reinterpret_cast<const u32x4*>(sp) + (int64_t)(f0 + i) * P * 4 + c4;
-  }
-
-  u32x4 wc[NW], sc[NW], wnx[NW], snx[NW];
-#pragma unroll
-  for (int j = 0; j < SJ; ++j) stg[j] = *reinterpret_cast<const u32x4*>(xsrc[j]);
-#pragma unroll
-  for (int i = 0; i < NW; ++i) {
-    wc[i] = wsrc[i][0];
-    sc[i] = ssrc[i][0];
-  }
-#pragma unroll
-  for (int j = 0; j < SJ; ++j) *reinterpret_cast<u32x4*>(&xl[0][sdst + 16 * j * XROW]) = stg[j];
-  lds_barrier();
-
-  f32x4 T[NW][MW];
-#pragma unroll
-  for (int i = 0; i < NW; ++i)
-#pragma unroll
-    for (int u = 0; u < MW; ++u) T[i][u] = (f32x4){0.f, 0.f, 0.f, 0.f};
-  const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
-  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-  uint32_t nib = 0x000F000Fu;
-  asm volatile("" : "+v"(nib));  // keep the nibble mask in a VGPR
-
-  // Straight-line stage body: the last stage reloads itself and writes the
-  // idle LDS buffer instead of branching (a branch around the prefetch made
-  // the compiler keep more registers live and cost 5%).
-  for (int p = 0; p < P; ++p) {
-    const int buf = p & 1;
-    const int pn = min(p + 1, P - 1);
-    {
-#pragma unroll
-      for (int j = 0; j < SJ; ++j)
-        stg[j] = *reinterpret_cast<const u32x4*>(xsrc[j] + pn * kStageK);
-#pragma unroll
-      for (int i = 0; i < NW; ++i) {
-        wnx[i] = wsrc[i][pn * 64];
-        snx[i] = ssrc[i][pn * 4];
-      }
-    }
-#pragma unroll
-    for (int gl = 0; gl < 2; ++gl) {
-      u32x4 X[MW][2];
-#pragma unroll
-      for (int u = 0; u < MW; ++u)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int row = (wm * MW + u) * 16 + r16;
-          const int ch = 8 * gl + 4 * h + c4;
-          X[u][h] = *reinterpret_cast<const u32x4*>(&xl[buf][row * XROW + ((ch ^ r16) << 4)]);
-        }
-      // X_g of the row fragments this wave owns (u % WN == wn)
-#pragma unroll
-      for (int u = 0; u < MW; ++u)
-        if (u % WN == wn) {
-          f32x4 a = mfma(ones, X[u][0], zero);
-          a = mfma(ones, X[u][1], a);
-          sx[(2 * p + gl) * MT + (wm * MW + u) * 16 + r16] = a[0];  // the 4 lane groups agree
-        }
-#pragma unroll
-      for (int i = 0; i < NW; ++i) {
-        const u32x4 A0 = unpack_w(wc[i][2 * gl], nib), A1 = unpack_w(wc[i][2 * gl + 1], nib);
-        float s[4];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) s[r] = gl ? bf_hi(sc[i][r]) : bf_lo(sc[i][r]);
-#pragma unroll
-        for (int u = 0; u < MW; ++u) {
-          f32x4 a = mfma(A0, X[u][0], zero);
-          a = mfma(A1, X[u][1], a);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) T[i][u][r] = fmaf(s[r], a[r], T[i][u][r]);
-        }
-      }
-    }
-    {
-#pragma unroll
-      for (int j = 0; j < SJ; ++j)
-        *reinterpret_cast<u32x4*>(&xl[buf ^ 1][sdst + 16 * j * XROW]) = stg[j];
-#pragma unroll
-      for (int i = 0; i < NW; ++i) {
-        wc[i] = wnx[i];
-        sc[i] = snx[i];
-      }
-    }
-    lds_barrier();
-  }
-
-  // sum_g (b_g - 128 s_g) X_g, X_g = hi + mid + lo exactly
-  for (int j = 0; j < G; j += 32) {
-    const bool gin = j + 8 * c4 < G;  // G is a multiple of 8
-#pragma unroll
-    for (int u = 0; u < MW; ++u) {
-      const int row = (wm * MW + u) * 16 + r16;
-      u32x4 hi, mid, lo;
-#pragma unroll
-      for (int e = 0; e < 8; e += 2) {
-        float v0 = 0.f, v1 = 0.f;
-        if (gin) {
-          v0 = sx[(j + 8 * c4 + e) * MT + row];
-          v1 = sx[(j + 8 * c4 + e + 1) * MT + row];
-        }
-        const uint32_t h = f2bf2(v0, v1);
-        const float r0 = v0 - bf_lo(h), r1 = v1 - bf_hi(h);
-        const uint32_t md = f2bf2(r0, r1);
-        hi[e >> 1] = h;
-        mid[e >> 1] = md;
-        lo[e >> 1] = f2bf2(r0 - bf_lo(md), r1 - bf_hi(md));
-      }
-#pragma unroll
-      for (int i = 0; i < NW; ++i) {
-        const int64_t n = (int64_t)(f0 + i) * 16 + r16;
-        u32x4 Ab = {0u, 0u, 0u, 0u}, As = {0u, 0u, 0u, 0u};
-        if (gin) {
-          Ab = *reinterpret_cast<const u32x4*>(bias + n * G + j + 8 * c4);
-          As = *reinterpret_cast<const u32x4*>(nsc + n * G + j + 8 * c4);
-        }
-        f32x4 t = T[i][u];
-        t = mfma(Ab, hi, t);
-        t = mfma(Ab, mid, t);
-        t = mfma(Ab, lo, t);
-        t = mfma(As, hi, t);
-        t = mfma(As, mid, t);
-        t = mfma(As, lo, t);
-        T[i][u] = t;
-      }
-    }
-  }
-
-#pragma unroll
-  for (int u = 0; u < MW; ++u) {
-    const int m = m0 + (wm * MW + u) * 16 + r16;
-#pragma unroll
-    for (int i = 0; i < NW; ++i) {
-      const int n = (f0 + i) * 16 + 4 * c4;
-      if (m < M && n < N) {
-        const f32x4 t = T[i][u];
-        *reinterpret_cast<u32x2*>(y + (int64_t)m * ys + n) = (u32x2){f2bf2(t[0], t[1]), f2bf2(t[2], t[3])};
-      }
-    }
-  }
+// Tile of work-group L among mt x nt (rows x columns of tiles). XCD L % 8 takes
+// a contiguous run of the tiles ordered in bands of 8 row tiles, column by
+// column inside a band, so that the groups which run side by side on an XCD
+// share 8 row tiles of x and as many column tiles of the weights in its L2.
+__device__ __forceinline__ void tile_of(int L, int mt, int nt, int& tm, int& tn) {
+  const int n = mt * nt, x = L & 7;
+  const int t = mt == 1 ? L : x * (n >> 3) + min(x, n & 7) + (L >> 3);
+  const int band = t / (8 * nt), rows = min(8, mt - 8 * band), r = t - band * 8 * nt;
+  tm = 8 * band + r % rows;
+  tn = r / rows;
 }
 
+// Split group sums of x's rows for the tile kernel: X_g[m] (by the ones-MFMA
+// that the tile kernel's own sums use, so the bits are the same) as three bf16
+// parts in xsg [ceil(M / 64)][3][64][G]. A wave takes 16 rows x 8 groups; the
+// call reads x once (16384 x 2048: about 20 us, bound by that read).
+__global__ __launch_bounds__(256) void qlinear_xsum_kernel(const uint16_t* __restrict__ x,
+                                                           int64_t xs, int M, int K,
+                                                           uint16_t* __restrict__ xsg) {
+  const int lane = threadIdx.x & 63, r16 = lane & 15, c4 = lane >> 4;
+  const int G = K >> 6, oct = G >> 3;
+  const int idx = blockIdx.x * 4 + (threadIdx.x >> 6);
+  const int rb = idx / oct, g0 = (idx - rb * oct) * 8;
+  if (16 * rb >= M) return;
+  const uint16_t* src = x + (int64_t)min(16 * rb + r16, M - 1) * xs + 64 * g0 + 8 * c4;
+  u32x4 X[8][2];
+#pragma unroll
+  for (int g = 0; g < 8; ++g)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) X[g][h] = *reinterpret_cast<const u32x4*>(src + 64 * g + 32 * h);
+  const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
+  float v0 = 0.f, v1 = 0.f;  // lane group c4 keeps groups 2 c4 and 2 c4 + 1
+#pragma unroll
+  for (int g = 0; g < 8; ++g) {
+    f32x4 a = mfma(ones, X[g][0], (f32x4){0.f, 0.f, 0.f, 0.f});
+    a = mfma(ones, X[g][1], a);
+    if (g & 1)
+      v1 = c4 == g >> 1 ? a[0] : v1;
+    else
+      v0 = c4 == g >> 1 ? a[0] : v0;
+  }
+  const uint32_t hi = f2bf2(v0, v1);
+  const float q0 = v0 - bf_lo(hi), q1 = v1 - bf_hi(hi);
+  const uint32_t mid = f2bf2(q0, q1);
+  const uint32_t lo = f2bf2(q0 - bf_lo(mid), q1 - bf_hi(mid));
+  uint16_t* dst = xsg + ((int64_t)(rb >> 2) * 3 * 64 + 16 * (rb & 3) + r16) * G + g0 + 2 * c4;
+  *reinterpret_cast<uint32_t*>(dst) = hi;
+  *reinterpret_cast<uint32_t*>(dst + 64 * G) = mid;
+  *reinterpret_cast<uint32_t*>(dst + 128 * G) = lo;
+}
 
-// Very wide layers at decode sizes (lm_head): 64 x 128 tiles of four waves in
-// a row, every wave with all 64 rows and two 16-column fragments (the weight
-// fragment is the MFMA A operand, as in qlinear_kernel). Per stage of 128 k:
+// 64 x 128 tiles of four waves in a row, every wave with all 64 rows and two
+// 16-column fragments (the weight fragment is the MFMA A operand: 16 n x 32 k,
+// the activations the B operand, so a lane ends with four consecutive n of one
+// row m). Takes prefill shapes (M > 64) and, at decode sizes, very wide layers
+// (lm_head). Per stage of 128 k:
 //  - x (64 rows x 256 B) is copied into LDS by DMA (buffer_load ... lds: wave
 //    w copies rows 4w + 16j .. +3, 1 KiB per load, lane L to byte 16 L of
 //    those rows, i.e. physical chunk L % 16 of row 4w + 16j + L / 16, which
-//    holds logical chunk (L % 16) ^ (row % 16) -- the swizzle of
-//    qlinear_kernel), double buffered;
+//    holds logical chunk (L % 16) ^ (row % 16): operand reads are
+//    conflict-free), double buffered;
 //  - the weights go to registers one stage ahead;
 //  - the scales (64 B per fragment) are copied into LDS by DMA, one 4-byte
 //    copy per wave for its two fragments: a 16-byte load per lane of the
 //    same block costs the vector memory path as much as a weight load.
-// Weights and scales are read through buffer resources with the stage in
-// soffset, so no address registers are kept per stage.
+// All of them are read through buffer resources that start at the tile's own
+// rows or fragments, with the stage in soffset, so no address registers are
+// kept per stage and offsets stay small at any size.
 // Each stage ends with this wave's copies of the next stage landed (vmcnt 0)
 // and a bare barrier: an LDS fence would also count the copies. The ring
 // slots are separate arrays, so that the compiler can tell copies into one
 // from reads of another.
-// Group sums X_g: wave w forms those of its own 16-row block with the
+// Group sums X_g. XS = 0: wave w forms those of its own 16-row block with the
 // ones-MFMA and keeps them in registers, lane group c4 holding group 4t + c4
-// of ring turn t (a shift register of KT values, KT >= G / 4); they are
+// of ring turn t (a shift register of KT values, KT >= groups / 4); they are
 // stored to LDS once after the loop. (An LDS store in the loop made the
-// compiler wait there for the DMA copies of the next stage.) With XS the
-// caller's split sums (xsg [3][64][G] bf16, launch_add_norm's) are copied
-// into LDS by DMA with the first stage instead, and no X_g products are
-// formed.
-// K a multiple of 512 (G a multiple of 8), G <= 4 KT; three waves per SIMD
-// for K <= 2048 (KT = 8), two above.
-template <int KT, bool XS>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KT <= 8 ? 3 : 2, KT <= 8 ? 3 : 2))) void qlinear_head_kernel(
+// compiler wait there for the DMA copies of the next stage.) XS = 1: the
+// caller's split sums (xsg [3][64][K/64] bf16, launch_add_norm's) are copied
+// into LDS by DMA with the first stage. XS = 2: split sums of every row tile
+// (xsg [tile][3][64][K/64], qlinear_xsum_kernel's) read where they are used.
+// K slices: work-group (tile, s) takes stages [s Ps, (s + 1) Ps); with several
+// slices it leaves its f32 tile (its groups' correction included) in part for
+// qlinear_tile_sum_kernel. Ps a multiple of 4, 2 Ps <= 4 KT.
+//
+// What bounds prefill: the issue of about 68 VALU instructions per wave and
+// group (one scale FMA per output, 7 unpacks per weight dword) beside 16
+// MFMAs, of which only a part overlaps, and the 8 KiB of operands per wave
+// and group from LDS. Three waves per SIMD hide the rest. 16384 x 2048 ->
+// 12,352: 880 us, 941 TFLOP/s (1,425 us for 32 x 64 wave tiles, two waves
+// per SIMD, x staged through registers); 16384 x 4096 -> 2048: 309 us (458).
+// 64-column waves (64 x 256 tiles, two waves per SIMD) took 871 and 304 us
+// there but 219 against 199 at M = 3688, where fewer tiles leave a last round
+// half empty.
+template <int KT, int XS>
+__global__ __launch_bounds__(256)
+    __attribute__((amdgpu_waves_per_eu(KT > 8 && XS == 1 ? 2 : 3, KT > 8 && XS == 1 ? 2 : 3))) void
+    qlinear_tile_kernel(
     const uint16_t* __restrict__ x, int64_t xs, int M, int K, const uint16_t* __restrict__ wp,
     const uint16_t* __restrict__ sp, const uint16_t* __restrict__ bias,
     const uint16_t* __restrict__ nsc, int N, int Npad, uint16_t* __restrict__ y, int64_t ys,
-    const uint16_t* __restrict__ xsg) {
+    const uint16_t* __restrict__ xsg, int Ps, float* __restrict__ part) {
   constexpr int MW = 4, NW = 2, MT = 64;
   constexpr int XROW = kStageK * 2;  // bytes per staged x row
   constexpr int GMAX = 4 * KT, GJ = GMAX / 32;
   static_assert(GMAX % 32 == 0, "whole 32-group chunks");
+  constexpr bool LATE = KT > 8 || XS == 2;  // correction operands loaded where they are used
   __shared__ __align__(16) uint8_t xl0[MT * XROW];
   __shared__ __align__(16) uint8_t xl1[MT * XROW];
   __shared__ __align__(16) uint8_t sl0[4 * 256];  // per wave: its fragments' 2 x 64 B
   __shared__ __align__(16) uint8_t sl1[4 * 256];
   // X_g: f32 [g][m] (formed here) or the caller's bf16 [3][m][G]
-  __shared__ __align__(16) uint8_t sxb[XS ? 3 * MT * GMAX * 2 : GMAX * MT * 4];
+  __shared__ __align__(16) uint8_t sxb[XS == 0 ? GMAX * MT * 4 : XS == 1 ? 3 * MT * GMAX * 2 : 16];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int G = K >> 6, P = K >> 7;
-  const int f0 = blockIdx.x * 8 + wave * NW;  // first column fragment of the wave
+  // stages of all K and of this work-group's slice [pofs, pofs + Ps); groups likewise
+  const int Gt = K >> 6, Pt = K >> 7, G = 2 * Ps;
+  const int pofs = blockIdx.y * Ps;
+  int tm, tn;
+  tile_of(blockIdx.x, (M + MT - 1) / MT, (Npad + 64 * NW - 1) / (64 * NW), tm, tn);
+  const int m0 = tm * MT;
+  const int fg = tn * 4 * NW;     // first column fragment of the work-group
+  const int f0 = fg + wave * NW;  // and of the wave
+  const int nfr = Npad / 16;
   const int r16 = lane & 15, c4 = lane >> 4;
 
-  const __amdgpu_buffer_rsrc_t xrs = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)x, (short)0, (int)(((int64_t)(M - 1) * xs + K) * 2), 0x00020000);
+  // The buffers of a tile: its weights and scales (fragments past Npad read as
+  // zeros) and, per x copy, the rows from its first one on (a lane past row
+  // M - 1 copies row M - 1 again; its outputs are not stored).
+  const int64_t left = min(nfr - fg, 4 * NW);
   const __amdgpu_buffer_rsrc_t wrs = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)wp, (short)0, (int)((int64_t)(Npad / 16) * P * 1024), 0x00020000);
+      (void*)(wp + (int64_t)fg * Pt * 512), (short)0, (int)(left * Pt * 1024), 0x00020000);
   const __amdgpu_buffer_rsrc_t srs = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)sp, (short)0, (int)((int64_t)(Npad / 16) * P * 64), 0x00020000);
+      (void*)(sp + (int64_t)fg * Pt * 32), (short)0, (int)(left * Pt * 64), 0x00020000);
+  __amdgpu_buffer_rsrc_t xrs[4];
   int xvo[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    const int row = 4 * (wave + 4 * j) + (lane >> 4);
-    xvo[j] = (int)((min(row, M - 1) * xs + 8 * ((lane & 15) ^ (row & 15))) * 2);
+    const int rb = 4 * (wave + 4 * j), r0 = min(m0 + rb, M - 1);
+    const int dr = min(m0 + rb + (lane >> 4), M - 1) - r0;
+    xrs[j] = __builtin_amdgcn_make_buffer_rsrc((void*)(x + (int64_t)r0 * xs), (short)0, -1, 0x00020000);
+    xvo[j] = (int)((uint32_t)(dr * xs * 2) + 16 * ((lane & 15) ^ ((rb + (lane >> 4)) & 15)));
   }
-  const int wvo0 = (f0 * P * 64 + lane) * 16, wvo1 = wvo0 + P * 1024;
-  // scale copy: lane L -> fragment f0 + (L % 32) / 16, dword L % 16 (lanes 32-63 repeat 0-31)
-  const int svo = ((f0 + ((lane & 31) >> 4)) * P * 64 + 4 * (lane & 15));
+  const int wvo = (wave * NW * Pt * 64 + lane) * 16;
+  // scale copy: lane L -> fragment f0 + (L / 16) % NW, dword L % 16
+  const int svo = (wave * NW + ((lane >> 4) & (NW - 1))) * Pt * 64 + 4 * (lane & 15);
 
   u32x4 w0[NW], w1[NW];  // the two weight register sets
   // stage p's loads into ring slot S: x, weights, scales (LB = 4 + NW + 1 loads)
-  auto batch = [&](int p, auto slot) {
+  auto batch = [&](int ps, auto slot) {
     constexpr int S = decltype(slot)::value;
+    const int p = pofs + ps;
     uint8_t* const xd = S ? xl1 : xl0;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          xrs, (void __attribute__((address_space(3)))*)(xd + 4 * (wave + 4 * j) * XROW), 16,
+          xrs[j], (void __attribute__((address_space(3)))*)(xd + 4 * (wave + 4 * j) * XROW), 16,
           xvo[j], p * XROW, 0, 0);
     u32x4* const wd = S ? w1 : w0;
-    wd[0] = __builtin_amdgcn_raw_buffer_load_b128(wrs, wvo0, p * 1024, 0);
-    wd[1] = __builtin_amdgcn_raw_buffer_load_b128(wrs, wvo1, p * 1024, 0);
+#pragma unroll
+    for (int i = 0; i < NW; ++i)
+      wd[i] = __builtin_amdgcn_raw_buffer_load_b128(wrs, wvo, (i * Pt + p) * 1024, 0);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(
         srs, (void __attribute__((address_space(3)))*)((S ? sl1 : sl0) + wave * 256), 4, svo,
         p * 64, 0, 0);
   };
   // correction operands b and -128 s of this wave's fragments (groups past G: zero)
   u32x4 Ab[NW][GJ], As[NW][GJ];
+  auto corr1 = [&](int i, int jb, u32x4& ab, u32x4& as) {
+    const bool gin = 32 * jb + 8 * c4 < G && f0 + i < nfr;
+    const int64_t o = gin ? (int64_t)((f0 + i) * 16 + r16) * Gt + 2 * pofs + 32 * jb + 8 * c4 : 0;
+    ab = *reinterpret_cast<const u32x4*>(bias + o);
+    as = *reinterpret_cast<const u32x4*>(nsc + o);
+    if (!gin) ab = as = (u32x4){0u, 0u, 0u, 0u};
+  };
   auto corr = [&]() {
 #pragma unroll
     for (int i = 0; i < NW; ++i)
 #pragma unroll
-      for (int jb = 0; jb < GJ; ++jb) {
-        const bool gin = 32 * jb + 8 * c4 < G;
-        const int64_t o = (int64_t)((f0 + i) * 16 + r16) * G + (gin ? 32 * jb + 8 * c4 : 0);
-        Ab[i][jb] = *reinterpret_cast<const u32x4*>(bias + o);
-        As[i][jb] = *reinterpret_cast<const u32x4*>(nsc + o);
-        if (!gin) Ab[i][jb] = As[i][jb] = (u32x4){0u, 0u, 0u, 0u};
-      }
+      for (int jb = 0; jb < GJ; ++jb) corr1(i, jb, Ab[i][jb], As[i][jb]);
   };
 
-  if constexpr (XS) {  // the caller's split sums, 3 x 64 rows x G bf16, in 1 KiB copies
+  if constexpr (XS == 1) {  // the caller's split sums, 3 x 64 rows x G bf16, in 1 KiB copies
     const __amdgpu_buffer_rsrc_t grs = __builtin_amdgcn_make_buffer_rsrc(
         (void*)xsg, (short)0, 3 * MT * G * 2, 0x00020000);
     for (int c = wave; c < (3 * MT * G * 2 + 1023) / 1024; c += 4)
@@ -429,7 +332,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KT <= 8 ? 3
     constexpr int S = decltype(slot)::value, kind = decltype(kindc)::value;
     constexpr bool last = decltype(lastc)::value;
     if constexpr (kind == 1) batch(p + 1, std::integral_constant<int, 1 - S>{});
-    if constexpr (kind == 2) corr();
+    if constexpr (kind == 2 && !LATE) corr();
     __builtin_amdgcn_sched_barrier(0);
     const uint8_t* const cur = S ? xl1 : xl0;
     const u32x4* const wc = S ? w1 : w0;
@@ -444,7 +347,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KT <= 8 ? 3
           const int ch = 8 * gl + 4 * h + c4;
           X[u][h] = *reinterpret_cast<const u32x4*>(&cur[row * XROW + ((ch ^ r16) << 4)]);
         }
-      if constexpr (!XS) {
+      if constexpr (XS == 0) {
         // X_g of group 2p + gl, rows 16 wave + r16: lane group c4 keeps it when
         // (2 S + gl) == c4, in the newest shift-register slot
 #pragma unroll
@@ -490,20 +393,20 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KT <= 8 ? 3
   using NL = std::false_type;
   int p = 0;
 #pragma nounroll
-  for (; p < P - 2; p += 2) {
-    if constexpr (!XS) shift();
+  for (; p < Ps - 2; p += 2) {
+    if constexpr (XS == 0) shift();
     stage(p, S0{}, S1{}, NL{});
     stage(p + 1, S1{}, S1{}, NL{});
   }
-  if constexpr (!XS) shift();
+  if constexpr (XS == 0) shift();
   stage(p, S0{}, S1{}, NL{});
   stage(p + 1, S1{}, K2{}, std::true_type{});
   wait_vm<0>();
   wait_lgkm0();
-  if constexpr (!XS) {
-    // turn t (of P / 2) sits in pk[KT - P/2 + t]: group 4t + c4 of rows 16 wave + r16
+  if constexpr (XS == 0) {
+    // turn t (of Ps / 2) sits in pk[KT - Ps/2 + t]: group 4t + c4 of rows 16 wave + r16
     float* const sx = reinterpret_cast<float*>(sxb);
-    const int k0 = KT - P / 2;
+    const int k0 = KT - Ps / 2;
 #pragma unroll
     for (int k = 0; k < KT; ++k)
       if (k >= k0) sx[(4 * (k - k0) + c4) * MT + wave * 16 + r16] = pk[k];
@@ -511,54 +414,81 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KT <= 8 ? 3
   lds_barrier();
 
   // sum_g (b_g - 128 s_g) X_g, X_g = hi + mid + lo exactly
-#pragma unroll
-  for (int u = 0; u < MW; ++u) {
+  auto split = [&](int u, int jb, u32x4& hi, u32x4& mid, u32x4& lo) {
     const int row = u * 16 + r16;
+    const bool gin = 32 * jb + 8 * c4 < G;
+    if constexpr (XS != 0) {
+      const uint16_t* const xsl =
+          XS == 1 ? reinterpret_cast<const uint16_t*>(sxb) : xsg + (int64_t)tm * 3 * MT * G;
+      const int o = row * G + (gin ? 32 * jb + 8 * c4 : 0);
+      hi = *reinterpret_cast<const u32x4*>(xsl + o);
+      mid = *reinterpret_cast<const u32x4*>(xsl + MT * G + o);
+      lo = *reinterpret_cast<const u32x4*>(xsl + 2 * MT * G + o);
+      if (!gin) hi = mid = lo = (u32x4){0u, 0u, 0u, 0u};
+    } else {
+      const float* const sx = reinterpret_cast<const float*>(sxb);
 #pragma unroll
-    for (int jb = 0; jb < GJ; ++jb) {
-      const bool gin = 32 * jb + 8 * c4 < G;
-      u32x4 hi, mid, lo;
-      if constexpr (XS) {
-        const uint16_t* const xsl = reinterpret_cast<const uint16_t*>(sxb);
-        const int o = row * G + (gin ? 32 * jb + 8 * c4 : 0);
-        hi = *reinterpret_cast<const u32x4*>(xsl + o);
-        mid = *reinterpret_cast<const u32x4*>(xsl + MT * G + o);
-        lo = *reinterpret_cast<const u32x4*>(xsl + 2 * MT * G + o);
-        if (!gin) hi = mid = lo = (u32x4){0u, 0u, 0u, 0u};
-      } else {
-        const float* const sx = reinterpret_cast<const float*>(sxb);
-#pragma unroll
-        for (int e = 0; e < 8; e += 2) {
-          float v0 = 0.f, v1 = 0.f;
-          if (gin) {
-            v0 = sx[(32 * jb + 8 * c4 + e) * MT + row];
-            v1 = sx[(32 * jb + 8 * c4 + e + 1) * MT + row];
-          }
-          const uint32_t h = f2bf2(v0, v1);
-          const float r0 = v0 - bf_lo(h), r1 = v1 - bf_hi(h);
-          const uint32_t md = f2bf2(r0, r1);
-          hi[e >> 1] = h;
-          mid[e >> 1] = md;
-          lo[e >> 1] = f2bf2(r0 - bf_lo(md), r1 - bf_hi(md));
+      for (int e = 0; e < 8; e += 2) {
+        float v0 = 0.f, v1 = 0.f;
+        if (gin) {
+          v0 = sx[(32 * jb + 8 * c4 + e) * MT + row];
+          v1 = sx[(32 * jb + 8 * c4 + e + 1) * MT + row];
         }
-      }
-#pragma unroll
-      for (int i = 0; i < NW; ++i) {
-        f32x4 t = T[i][u];
-        t = mfma(Ab[i][jb], hi, t);
-        t = mfma(Ab[i][jb], mid, t);
-        t = mfma(Ab[i][jb], lo, t);
-        t = mfma(As[i][jb], hi, t);
-        t = mfma(As[i][jb], mid, t);
-        t = mfma(As[i][jb], lo, t);
-        T[i][u] = t;
+        const uint32_t h = f2bf2(v0, v1);
+        const float r0 = v0 - bf_lo(h), r1 = v1 - bf_hi(h);
+        const uint32_t md = f2bf2(r0, r1);
+        hi[e >> 1] = h;
+        mid[e >> 1] = md;
+        lo[e >> 1] = f2bf2(r0 - bf_lo(md), r1 - bf_hi(md));
       }
     }
+  };
+  auto correct = [&](f32x4& t, u32x4 ab, u32x4 as, u32x4 hi, u32x4 mid, u32x4 lo) {
+    t = mfma(ab, hi, t);
+    t = mfma(ab, mid, t);
+    t = mfma(ab, lo, t);
+    t = mfma(as, hi, t);
+    t = mfma(as, mid, t);
+    t = mfma(as, lo, t);
+  };
+  if constexpr (LATE) {
+#pragma nounroll
+    for (int jb = 0; jb < (G + 31) / 32; ++jb) {
+      u32x4 hi[MW], mid[MW], lo[MW];
+#pragma unroll
+      for (int u = 0; u < MW; ++u) split(u, jb, hi[u], mid[u], lo[u]);
+#pragma unroll
+      for (int i = 0; i < NW; ++i) {
+        u32x4 ab, as;
+        corr1(i, jb, ab, as);
+#pragma unroll
+        for (int u = 0; u < MW; ++u) correct(T[i][u], ab, as, hi[u], mid[u], lo[u]);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < MW; ++u)
+#pragma unroll
+      for (int jb = 0; jb < GJ; ++jb) {
+        u32x4 hi, mid, lo;
+        split(u, jb, hi, mid, lo);
+#pragma unroll
+        for (int i = 0; i < NW; ++i) correct(T[i][u], Ab[i][jb], As[i][jb], hi, mid, lo);
+      }
   }
 
+  if (part != nullptr) {  // this slice's sums, for qlinear_tile_sum_kernel
+    f32x4* const pt = reinterpret_cast<f32x4*>(part) +
+                      ((int64_t)blockIdx.y * gridDim.x + blockIdx.x) * (MT * 128 / 4);
+#pragma unroll
+    for (int i = 0; i < NW; ++i)
+#pragma unroll
+      for (int u = 0; u < MW; ++u) pt[((wave * NW + i) * MW + u) * 64 + lane] = T[i][u];
+    return;
+  }
 #pragma unroll
   for (int u = 0; u < MW; ++u) {
-    const int m = u * 16 + r16;
+    const int m = m0 + u * 16 + r16;
 #pragma unroll
     for (int i = 0; i < NW; ++i) {
       const int n = (f0 + i) * 16 + 4 * c4;
@@ -568,6 +498,23 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(KT <= 8 ? 3
       }
     }
   }
+}
+
+// y = bf16(the K slices' tiles of qlinear_tile_kernel added in slice order).
+// grid (tiles, 8), block 256: thread (wave fragment, row block, lane) of a tile.
+__global__ __launch_bounds__(256) void qlinear_tile_sum_kernel(const float* __restrict__ part,
+                                                               int slices, int M, int N, int Npad,
+                                                               uint16_t* __restrict__ y, int64_t ys) {
+  const int e = blockIdx.y * 256 + threadIdx.x;  // ((fragment * 4 + u) * 64 + lane)
+  const f32x4* src = reinterpret_cast<const f32x4*>(part) + (int64_t)blockIdx.x * 2048 + e;
+  int tm, tn;
+  tile_of(blockIdx.x, (M + 63) / 64, Npad / 128, tm, tn);
+  const int lane = e & 63, u = (e >> 6) & 3, f = e >> 8;
+  const int m = tm * 64 + u * 16 + (lane & 15), n = tn * 128 + f * 16 + 4 * (lane >> 4);
+  if (m >= M || n >= N) return;
+  f32x4 t = src[0];
+  for (int s = 1; s < slices; ++s) t += src[(int64_t)s * gridDim.x * 2048];
+  *reinterpret_cast<u32x2*>(y + (int64_t)m * ys + n) = (u32x2){f2bf2(t[0], t[1]), f2bf2(t[2], t[3])};
 }
 
 // Decode shapes (M <= 64). A work-group owns 64 columns (four 16-wide
@@ -850,21 +797,18 @@ __global__ __launch_bounds__(256) void qlinear_sum_kernel(const float* __restric
   *reinterpret_cast<u32x2*>(y + (int64_t)m * ys + n) = (u32x2){f2bf2(t[0], t[1]), f2bf2(t[2], t[3])};
 }
 
-template <int MW, int NW, int WM, int WN>
-hipError_t launch_cfg(const QLinearArgs& a) {
-  constexpr int MT = 16 * MW * WM, NT = 16 * NW * WN;
-  const dim3 grid(a.Npad / NT, (a.M + MT - 1) / MT);
-  hipLaunchKernelGGL((qlinear_kernel<MW, NW, WM, WN>), grid, dim3(256), 0, a.stream, a.x, a.xs,
-                     a.M, a.K, reinterpret_cast<const u32x4*>(a.wp), a.sp, a.bias, a.nsc, a.N,
-                     a.y, a.ys);
-  return hipGetLastError();
-}
-
-template <int KT, bool XS>
-hipError_t launch_head(const QLinearArgs& a) {
-  hipLaunchKernelGGL((qlinear_head_kernel<KT, XS>), dim3(a.Npad / 128), dim3(256), 0, a.stream, a.x,
-                     a.xs, a.M, a.K, reinterpret_cast<const uint16_t*>(a.wp), a.sp, a.bias, a.nsc,
-                     a.N, a.Npad, a.y, a.ys, a.xsplit);
+template <int KT, int XS>
+hipError_t launch_tile(const QLinearArgs& a, int slices = 1) {
+  const int64_t tiles = (int64_t)((a.M + 63) / 64) * (a.Npad / 128);
+  if (tiles > INT32_MAX) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((qlinear_tile_kernel<KT, XS>), dim3((unsigned)tiles, slices), dim3(256), 0,
+                     a.stream, a.x, a.xs, a.M, a.K, reinterpret_cast<const uint16_t*>(a.wp), a.sp,
+                     a.bias, a.nsc, a.N, a.Npad, a.y, a.ys, a.xsplit, a.K / 128 / slices,
+                     slices > 1 ? a.part : nullptr);
+  hipError_t e = hipGetLastError();
+  if (e != hipSuccess || slices == 1) return e;
+  hipLaunchKernelGGL(qlinear_tile_sum_kernel, dim3((unsigned)tiles, 8), dim3(256), 0, a.stream, a.part,
+                     slices, a.M, a.N, a.Npad, a.y, a.ys);
   return hipGetLastError();
 }
 
@@ -887,16 +831,27 @@ int qlinear_decode_slices(int K, int Npad) {
   return K % 1024 == 0 ? K / 1024 : K / 512;
 }
 
+// K slices of a tile-kernel call of `tiles` 64 x 128 tiles. A work-group runs its
+// stages one after the other at about 1 us each while the chip is not full, so
+// a call with few tiles is cut along K: into the most slices that keep four
+// stages (512 k, whole sets of 8 groups) each and at most kQLinearPartTiles
+// work-groups. The slice sum is a launch of its own (3-4 us), which two slices
+// of 16 stages (K = 2048) do not pay back. Measured, unsliced against sliced:
+// K = 4096, N = 2048: M = 65 32.5 / 12.6 us (8 slices), 300 33.1 / 18.6 (4),
+// 1000 33.5 / 29.2 (2); K = 2048, N = 12,352, M = 100: 18.4 / 19.5 (2, not taken).
+int qlinear_tile_slices(int K, int64_t tiles) {
+  const int q = K / 512;
+  for (int s = q < 8 ? q : 8; s > (K <= 2048 ? 2 : 1); --s)
+    if (q % s == 0 && tiles * s <= kQLinearPartTiles) return s;
+  return 1;
+}
+
 // Tile choice: up to 64 rows (batched decode) qlinear_decode_kernel, whole K
 // (K = 512, 1024, 2048) or K slices (narrow layers, and every K above 2048 --
-// those always get a workspace); otherwise 64 x 128 tiles (prefill). Of the
-// tilings swept at 16384 x 2048 -> 12352 (four waves each, 16-wide fragments
-// per wave m x n: 4x4, 2x4, 4x2, 2x2, 2x4 in one row of waves, 1x4, 2x2 in
-// one column), 2 x 4 fragments per wave in a 2 x 2 wave grid was fastest:
-// about 200 VGPRs and 48 KB of LDS give two waves per SIMD (1.42 ms; 4 x 4
-// with one wave per SIMD took 1.98 ms). Deeper x prefetch (two stages in
-// registers) pushed it to one wave per SIMD and 2.06 ms; an XCD-aware tile
-// order (each XCD's L2 holding its own weight columns) changed nothing.
+// those always get a workspace); otherwise (prefill, and lm_head's decode
+// sizes) qlinear_tile_kernel's 64 x 128 tiles, cut along K where they are few
+// (qlinear_tile_slices), with the group sums formed once up front where they
+// are many (kSumTiles, kSumColumns).
 //
 // Decode kernel shapes (64 x 12352 x 2048 and 64 x 2048 x 4096, 30 distinct
 // layers): eight waves of two stages for K = 2048 (four waves of four stages,
@@ -913,7 +868,7 @@ int qlinear_decode_slices(int K, int Npad) {
 // with x copied by DMA at three waves per SIMD took 128-130 us timed alone
 // (142.7 for the register-staged form in the same harness; 137 with DMA at two
 // waves per SIMD; the register-staged form forced to three waves spills and
-// takes 182). qlinear_head_kernel, the DMA tile with its group sums kept in
+// takes 182). qlinear_tile_kernel, the DMA tile with its group sums kept in
 // registers through the K loop and its scales copied by DMA, takes 94-96 us
 // timed alone on weights that stream from HBM (106-112 for the DMA tile that
 // stored the sums to LDS in the loop, on the same boxes), 90 us in the
@@ -922,12 +877,9 @@ int qlinear_decode_slices(int K, int Npad) {
 hipError_t launch_qlinear(const QLinearArgs& a) {
   if (a.defer) *a.defer = QPartial{};
   if (a.M <= 64 && a.Npad >= kWideDecodeN) {
-    // buffer offsets of the packed weights are 32-bit; K is a multiple of 512
-    if (a.K % 512 != 0 || a.K > 4096 || (int64_t)a.Npad * a.K / 2 > INT32_MAX)
-      return launch_cfg<4, 2, 1, 4>(a);
     const bool xs = a.xsplit != nullptr;
-    if (a.K <= 2048) return xs ? launch_head<8, true>(a) : launch_head<8, false>(a);
-    return xs ? launch_head<16, true>(a) : launch_head<16, false>(a);
+    if (a.K <= 2048) return xs ? launch_tile<8, 1>(a) : launch_tile<8, 0>(a);
+    return xs ? launch_tile<16, 1>(a) : launch_tile<16, 0>(a);
   }
   if (a.M <= 64) {
     const int ns = a.part ? qlinear_decode_slices(a.K, a.Npad) : 1;
@@ -955,7 +907,26 @@ hipError_t launch_qlinear(const QLinearArgs& a) {
       return hipGetLastError();
     }
   }
-  return launch_cfg<2, 4, 2, 2>(a);
+  const int64_t tiles = (int64_t)((a.M + 63) / 64) * (a.Npad / 128);
+  const int slices = qlinear_tile_slices(a.K, tiles);
+  if (slices > 1 || tiles < kSumTiles || a.Npad < kSumColumns) {
+    if (a.K / slices <= 2048) return launch_tile<8, 0>(a, slices);
+    return launch_tile<16, 0>(a, slices);
+  }
+  QLinearArgs c = a;
+  for (int m = 0; m < a.M; m += kQLinearSumRows) {
+    c.M = a.M - m < kQLinearSumRows ? a.M - m : kQLinearSumRows;
+    c.x = a.x + m * a.xs;
+    c.y = a.y + m * a.ys;
+    const int waves = (c.M + 15) / 16 * (a.K / 512);
+    hipLaunchKernelGGL(qlinear_xsum_kernel, dim3((waves + 3) / 4), dim3(256), 0, a.stream, c.x, c.xs,
+                       c.M, c.K, a.xsum);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    c.xsplit = a.xsum;
+    if ((e = launch_tile<8, 2>(c)) != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace gdn

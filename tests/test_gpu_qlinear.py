@@ -166,6 +166,44 @@ def test_qlinear_prefill_rows_sampled(gpu):
     layer.close()
 
 
+@pytest.mark.parametrize("M,K,N", [
+    (65, 1536, 400),      # 3 slices of 4 stages, two row tiles, columns not a tile multiple
+    (128, 4096, 2048),    # whole row tiles, 8 slices
+    (321, 4096, 2048),    # 4 slices (96 tiles), one row in the last row tile
+    (1000, 4096, 2064),   # no slice: 272 tiles; 2,064 columns leave 16 in the last tile
+    (960, 4096, 2048),    # 2 slices (240 tiles)
+    (65, 2048, 9216),     # K = 2048: two slices would fit and are not taken
+    (2241, 4096, 8208),   # up-front group sums of 64 groups, one row in the last row tile
+    (16449, 512, 4112),   # more rows than one piece of the up-front sums
+])
+def test_qlinear_tiles_and_slices_sampled(gpu, M, K, N):
+    """The tile kernel's K slices and up-front group sums at the edges of
+    their rules, against the oracle at sampled rows and columns (the first,
+    the last and those beside the tile edges among them); x rows and y rows
+    are wider than K and N, and nothing past N is written."""
+    import torch
+    say("gdn_qlinear_forward", f"tiles M={M} K={K} N={N}")
+    rng = np.random.default_rng(505 + M)
+    w = rng.integers(0, 2**32, (N, K // 8), dtype=np.uint32)
+    s = O.f32_to_bf16((rng.random((N, K // 64)) * 0.004 + 0.001).astype(np.float32))
+    b = O.f32_to_bf16((rng.standard_normal((N, K // 64)) * 0.03).astype(np.float32))
+    x = np.zeros((M, K + 8), np.uint16)
+    x[:, :K] = O.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32))
+    layer = _layer(K, [(w, s, b)])
+    y = torch.full((M, N + 4), -1, dtype=torch.int16, device=gpu)
+    layer.forward(dev(x)[:, :K], y)
+    torch.cuda.synchronize()
+    yh = host(y)
+    assert np.all(yh[:, N:] == 0xFFFF), "columns past N were written"
+    edge = lambda n, t: {0, n - 1, *(i for k in range(t, n, t) for i in (k - 1, k))}  # noqa: E731
+    pick = lambda n, t, m: np.array(sorted(set(rng.choice(n, min(n, m), replace=False).tolist())  # noqa: E731
+                                           | set(sorted(edge(n, t))[:16]) | {n - 1}))
+    rows, cols = pick(M, 64, 64), pick(N, 128, 256)
+    yr, ye, mag = O.qmatmul_w4(x[rows, :K], w[cols], s[cols], b[cols])
+    _check(yh[np.ix_(rows, cols)], ye, mag, yr, f"qlinear tiles M={M} K={K} N={N}")
+    layer.close()
+
+
 def test_qlinear_output_feeds_gated_decode_in_place(gpu):
     """Hidden states -> merged q|k|v|z|b|a projection -> gdn_decode_gated reading
     qkvz and ab as column slices of the one output (no copies), against the
