@@ -7,14 +7,9 @@
 // channel it reads: no two work-groups touch the same conv-state bytes of a
 // slot.
 //
-// The recurrence kernel (prepared q/k/v, T tokens) holds each 128x128 f32
-// tile in a "tile team" of 256 threads, 64 floats per thread:
-//   lt = thread index in the team, grp = lt >> 3 (0..31), sub = lt & 7;
-//   rows  dv = grp + 32*i            (i = 0..3)
-//   cols  dk = 4*(sub + 8*j) + e     (j = 0..3, e = 0..3)
-// and reduces over dk inside 8 aligned lanes (three DPP adds, sum8). The
-// fused decode kernel uses a row layout with 16 lanes per row instead (see
-// decode_kernel).
+// The recurrence kernel (prepared q/k/v, T tokens) splits a head's rows over
+// independent waves (see recurrent_kernel). The fused decode kernel uses a row
+// layout with 16 lanes per row (see decode_kernel).
 //
 // Arithmetic (metal_gdn.rs:37-62): s *= g; kv = s.k; d = (v - kv)*beta;
 // s += k d; y = s.q. The readout is taken from the decayed state in the same
@@ -25,75 +20,8 @@
 
 namespace gdn {
 
-struct TileRegs {
-  v4f s[4][4];
-};
-
-// slot: the slot's state (Hv * Dv * Dk floats); rows of value head hv are
-// addressed through state_row_offset.
-__device__ __forceinline__ void tile_load(TileRegs& t, const float* __restrict__ slot, int hv,
-                                          int Hk, int R, int grp, int sub) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const float* row = slot + state_row_offset(hv, grp + 32 * i, Hk, R);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      t.s[i][j] = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(row + 4 * (sub + 8 * j)));
-  }
-}
-
-__device__ __forceinline__ void tile_store(const TileRegs& t, float* __restrict__ slot, int hv,
-                                           int Hk, int R, int grp, int sub) {
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    float* row = slot + state_row_offset(hv, grp + 32 * i, Hk, R);
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      __builtin_nontemporal_store(t.s[i][j], reinterpret_cast<v4f*>(row + 4 * (sub + 8 * j)));
-  }
-}
-
 __device__ __forceinline__ float dot4(const v4f& a, const v4f& b) {
   return a.x * b.x + a.y * b.y + a.z * b.z + a.w * b.w;
-}
-
-// One token on the register tile. kl/ql: k and q of the token in LDS (Dk
-// floats each); vrow[i]: v at row grp+32i; kq = k.q over all of Dk. yrow[i]
-// gets the output of row grp+32i (identical in the 8 lanes of a row group).
-// k/q are read from LDS per column block (j outer) so that only 8 of them are
-// live at a time; the compiler barrier between the passes makes the second
-// pass re-read k instead of keeping 16 registers alive across the reduction.
-__device__ __forceinline__ void tile_step(TileRegs& t, const float* kl, const float* ql, int sub,
-                                          const float vrow[4], float g, float beta, float kq,
-                                          float yrow[4]) {
-  float kd[4] = {0.f, 0.f, 0.f, 0.f}, qd[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const v4f kj = *reinterpret_cast<const v4f*>(kl + 4 * (sub + 8 * j));
-    const v4f qj = *reinterpret_cast<const v4f*>(ql + 4 * (sub + 8 * j));
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const v4f sv = t.s[i][j] * g;
-      kd[i] += dot4(sv, kj);
-      qd[i] += dot4(sv, qj);
-      t.s[i][j] = sv;
-    }
-  }
-  float delta[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    kd[i] = sum8(kd[i]);
-    qd[i] = sum8(qd[i]);
-    delta[i] = (vrow[i] - kd[i]) * beta;
-    yrow[i] = qd[i] + delta[i] * kq;
-  }
-  asm volatile("" ::: "memory");
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const v4f kj = *reinterpret_cast<const v4f*>(kl + 4 * (sub + 8 * j));
-#pragma unroll
-    for (int i = 0; i < 4; ++i) t.s[i][j] += kj * delta[i];
-  }
 }
 
 // Baked rms-norm weights (qwen3_5.rs:551-552): bf16(1/128) and bf16(128^-0.5).
@@ -101,67 +29,142 @@ constexpr float kQNormW = 0.0078125f;
 constexpr float kKNormW = 0.08837890625f;
 constexpr float kNormEps = 1e-6f;
 
+// Item of work-group L among n: XCD x = L % 8 takes items
+// [x*(n/8) + min(x, n%8), ...) in order, one per group it receives.
+__device__ __forceinline__ int xcd_item(int L, int n) {
+  const int x = L & 7;
+  return x * (n >> 3) + min(x, n & 7) + (L >> 3);
+}
+
 // -------------------------------------------------------------------------
 // Recurrence on prepared q/k/v/g/beta for T tokens per sequence (the
 // gated_delta_kernel contract, metal_gdn.rs:10-67), state in pool slots.
-// grid (Hk, B), block 256*R.
-template <int R>
-__global__ __launch_bounds__(256 * R) void recurrent_kernel(
+//
+// A wave owns 8 NI rows of one (sequence, value head) and keeps them in
+// registers for all T tokens: lane = 8 grp + sub, thread row i is
+// 8 (NI w + i) + grp of the head (w the wave's index in it), columns
+// 4 (sub + 8 j) + e; a dk-reduction is three DPP adds over 8 lanes. The rows of
+// a head need nothing of each other, so waves share nothing: each lane loads
+// its own 16 columns of k and q (the 8 row groups of a wave read the same
+// addresses), rec_ahead tokens ahead in registers, and there is no LDS and no
+// barrier. What bounds it is the serial chain of tokens: about 75 VALU
+// instructions per row and 50 for a token's conversions and k.q, at one wave
+// per SIMD. So NI is the largest of 4, 2, 1 that still gives every SIMD a wave.
+// 16/32 heads, T = 37: B = 1 18 us, B = 4 24 us (66 and 67 with one 512-thread
+// group per key head, four rows a thread, each token's inputs loaded and passed
+// through LDS between two barriers); B = 64, T = 64: 319 us (591).
+// tokens in flight per wave: enough to cover a load's latency at NI's pace
+__host__ __device__ constexpr int rec_ahead(int ni) { return ni == 4 ? 2 : 4; }
+
+// q and k rows are only known to be 2-byte aligned
+typedef uint32_t u32x2_a2 __attribute__((ext_vector_type(2), aligned(2)));
+
+template <int NI>
+struct RecToken {
+  u32x2_a2 k[4], q[4];
+  uint16_t v[NI], beta;
+  float g;
+};
+
+template <int R, int NI>
+__global__ __launch_bounds__(256) void recurrent_kernel(
     float* __restrict__ state, const int32_t* __restrict__ slot_ids, int num_slots, int Hk, int T,
     const uint16_t* __restrict__ q, const uint16_t* __restrict__ k,
     const uint16_t* __restrict__ v, const float* __restrict__ g,
     const uint16_t* __restrict__ beta, uint16_t* __restrict__ y, uint32_t* __restrict__ status) {
-  constexpr int NT = 256 * R;
-  const int hk = blockIdx.x, b = blockIdx.y;
+  constexpr int WPH = kDv / (8 * NI);  // waves per head
+  constexpr int kAhead = rec_ahead(NI);
   const int Hv = Hk * R;
-  const int tid = threadIdx.x;
+  const int wid = __builtin_amdgcn_readfirstlane(
+      xcd_item(blockIdx.x, gridDim.x) * 4 + (threadIdx.x >> 6));
+  const int head = wid / WPH, w = wid - head * WPH;
+  const int b = head / Hv, hv = head - b * Hv, hk = hv / R;
+  const int lane = threadIdx.x & 63, grp = lane >> 3, sub = lane & 7;
   const int slot = slot_ids[b];
   if ((unsigned)slot >= (unsigned)num_slots) {
-    if (tid == 0) flag_status(status, GDN_FLAG_BAD_SLOT);
+    if (lane == 0) flag_status(status, GDN_FLAG_BAD_SLOT);
     return;
   }
-  __shared__ __align__(16) float qs[kDk];
-  __shared__ __align__(16) float ks[kDk];
-  __shared__ float vs[R * kDv];
-  __shared__ float red[2];
-  __shared__ float gg[R], bb[R];
-
-  const int r = tid >> 8;
-  const int lt = tid & 255, grp = lt >> 3, sub = lt & 7;
-  const int hv = hk * R + r;
-  const int wave = tid >> 6, lane = tid & 63;
   float* sslot = state + (size_t)slot * Hv * kTileElems;
-  TileRegs t;
-  tile_load(t, sslot, hv, Hk, R, grp, sub);
-
-  for (int tt = 0; tt < T; ++tt) {
-    const size_t tok = (size_t)b * T + tt;
-    if (tid < kDk) {
-      const float qv = bf2f(q[(tok * Hk + hk) * kDk + tid]);
-      const float kv = bf2f(k[(tok * Hk + hk) * kDk + tid]);
-      qs[tid] = qv;
-      ks[tid] = kv;
-      const float p = wave_sum(qv * kv);
-      if (lane == 0) red[wave] = p;
-    }
-    for (int c = tid; c < R * kDv; c += NT) vs[c] = bf2f(v[(tok * Hv + hk * R) * kDv + c]);
-    if (tid < R) {
-      gg[tid] = g[tok * Hv + hk * R + tid];
-      bb[tid] = bf2f(beta[tok * Hv + hk * R + tid]);
-    }
-    __syncthreads();
-    const float kq = red[0] + red[1];
-    float vrow[4], yrow[4];
+  float* rows[NI];
+  v4f st[NI][4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) vrow[i] = vs[r * kDv + grp + 32 * i];
-    tile_step(t, ks, qs, sub, vrow, gg[r], bb[r], kq, yrow);
-    uint16_t* yo = y + (tok * Hv + hv) * kDv;
+  for (int i = 0; i < NI; ++i) {
+    rows[i] = sslot + state_row_offset(hv, 8 * (NI * w + i) + grp, Hk, R) + 4 * sub;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      if (sub == i) yo[grp + 32 * i] = f2bf(yrow[i]);
-    __syncthreads();
+    for (int j = 0; j < 4; ++j)
+      st[i][j] = __builtin_nontemporal_load(reinterpret_cast<const v4f*>(rows[i] + 32 * j));
   }
-  tile_store(t, sslot, hv, Hk, R, grp, sub);
+  const size_t tok0 = (size_t)b * T;
+  const uint16_t* kp = k + (tok0 * Hk + hk) * kDk + 4 * sub;
+  const uint16_t* qp = q + (tok0 * Hk + hk) * kDk + 4 * sub;
+  const uint16_t* vp = v + (tok0 * Hv + hv) * kDv + 8 * NI * w + grp;
+  uint16_t* yp = y + (tok0 * Hv + hv) * kDv + 8 * NI * w + grp;
+  const float* gp = g + tok0 * Hv + hv;
+  const uint16_t* bp = beta + tok0 * Hv + hv;
+  auto load = [&](int t, RecToken<NI>& x) {
+    const size_t o = (size_t)min(t, T - 1);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      x.k[j] = *reinterpret_cast<const u32x2_a2*>(kp + o * Hk * kDk + 32 * j);
+      x.q[j] = *reinterpret_cast<const u32x2_a2*>(qp + o * Hk * kDk + 32 * j);
+    }
+#pragma unroll
+    for (int i = 0; i < NI; ++i) x.v[i] = vp[o * Hv * kDv + 8 * i];
+    x.g = gp[o * Hv];
+    x.beta = bp[o * Hv];
+  };
+  auto unpack = [](u32x2_a2 u) { return (v4f){bf_lo(u.x), bf_hi(u.x), bf_lo(u.y), bf_hi(u.y)}; };
+  auto step = [&](int t, const RecToken<NI>& x) {
+    v4f kf[4], qf[4];
+    float kq = 0.f, kd[NI], qd[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) kd[i] = qd[i] = 0.f;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      kf[j] = unpack(x.k[j]);
+      qf[j] = unpack(x.q[j]);
+      kq += dot4(kf[j], qf[j]);
+#pragma unroll
+      for (int i = 0; i < NI; ++i) {
+        st[i][j] *= x.g;
+        kd[i] += dot4(st[i][j], kf[j]);
+        qd[i] += dot4(st[i][j], qf[j]);
+      }
+    }
+    kq = sum8(kq);
+    const float bt = bf2f(x.beta);
+    float yo = 0.f;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const float d = (bf2f(x.v[i]) - sum8(kd[i])) * bt;
+      const float yi = sum8(qd[i]) + d * kq;
+      yo = sub == i ? yi : yo;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) st[i][j] += kf[j] * d;
+    }
+    if (sub < NI) yp[(size_t)t * Hv * kDv + 8 * sub] = f2bf(yo);
+  };
+  RecToken<NI> x[kAhead];
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u) load(u, x[u]);
+  int t = 0;
+  for (; t + kAhead <= T; t += kAhead) {
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      step(t + u, x[u]);
+      load(t + u + kAhead, x[u]);
+      __builtin_amdgcn_sched_barrier(0);  // no token's conversions ahead of its turn
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < kAhead; ++u)
+    if (t + u < T) step(t + u, x[u]);
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      __builtin_nontemporal_store(st[i][j], reinterpret_cast<v4f*>(rows[i] + 32 * j));
 }
 
 // -------------------------------------------------------------------------
@@ -208,13 +211,6 @@ __device__ __forceinline__ float conv1(uint16_t c0, uint16_t c1, uint16_t c2, ui
 // Gap between a wave's state load pairs in the fused decode, in units of 64
 // clocks (s_sleep).
 constexpr int kDecodeLoadGap = 4;
-
-// Item of work-group L among n: XCD x = L % 8 takes items
-// [x*(n/8) + min(x, n%8), ...) in order, one per group it receives.
-__device__ __forceinline__ int xcd_item(int L, int n) {
-  const int x = L & 7;
-  return x * (n >> 3) + min(x, n & 7) + (L >> 3);
-}
 
 template <int R, bool GATED>
 __global__ __launch_bounds__(256 * R) void decode_kernel(
@@ -407,15 +403,13 @@ constexpr size_t kDecodeOccupancyLds = 80 * 1024;
 template <int R>
 static hipError_t launch_decode_r(const DecodeArgs& a) {
   const size_t lds = R == 2 ? kDecodeOccupancyLds : 0;
-  if (a.out)
-    hipLaunchKernelGGL((decode_kernel<R, true>), dim3(a.Hk * a.B), dim3(256 * R), lds, a.stream,
-                       a.state, a.conv, a.slot_ids, a.num_slots, a.Hk, a.mixed, a.xstride, a.ab, a.ab_stride,
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(a.Hk * a.B), dim3(256 * R), lds, a.stream, a.state, a.conv,
+                       a.slot_ids, a.num_slots, a.Hk, a.mixed, a.xstride, a.ab, a.ab_stride,
                        a.A_log, a.dt_bias, a.conv_w, a.y, a.norm_w, a.norm_eps, a.out, a.status);
-  else
-    hipLaunchKernelGGL((decode_kernel<R, false>), dim3(a.Hk * a.B), dim3(256 * R), lds, a.stream,
-                       a.state, a.conv, a.slot_ids, a.num_slots, a.Hk, a.mixed, a.xstride, a.ab, a.ab_stride,
-                       a.A_log, a.dt_bias, a.conv_w, a.y, a.norm_w, a.norm_eps, a.out, a.status);
-  return hipGetLastError();
+    return hipGetLastError();
+  };
+  return a.out ? go(decode_kernel<R, true>) : go(decode_kernel<R, false>);
 }
 
 hipError_t launch_decode(const DecodeArgs& a) {
@@ -427,11 +421,23 @@ hipError_t launch_decode(const DecodeArgs& a) {
   }
 }
 
+// Rows per thread: the fewest waves that still put one on each of the 1,024
+// SIMDs (B Hv heads of 16 / NI waves); more rows a thread share a token's
+// conversions, fewer spread its chain over idle SIMDs.
 template <int R>
 static hipError_t launch_recurrent_r(const RecurrentArgs& a) {
-  dim3 grid(a.Hk, a.B);
-  hipLaunchKernelGGL(recurrent_kernel<R>, grid, dim3(256 * R), 0, a.stream, a.state, a.slot_ids,
-                     a.num_slots, a.Hk, a.T, a.q, a.k, a.v, a.g, a.beta, a.y, a.status);
+  const int64_t heads = (int64_t)a.B * a.Hk * R;
+  auto go = [&](auto kern, int ni) {
+    hipLaunchKernelGGL(kern, dim3((unsigned)(heads * (16 / ni) / 4)), dim3(256), 0, a.stream, a.state,
+                       a.slot_ids, a.num_slots, a.Hk, a.T, a.q, a.k, a.v, a.g, a.beta, a.y,
+                       a.status);
+  };
+  if (heads * 4 >= 1024)
+    go(recurrent_kernel<R, 4>, 4);
+  else if (heads * 8 >= 1024)
+    go(recurrent_kernel<R, 2>, 2);
+  else
+    go(recurrent_kernel<R, 1>, 1);
   return hipGetLastError();
 }
 

@@ -146,6 +146,56 @@ def test_recurrent_matches_oracle(gpu, B, T):
     assert pool.check() == 0
 
 
+@pytest.mark.parametrize("B,T,Hk,Hv,off", [
+    (1, 1, 16, 32, 0),    # one row a thread, fewer tokens than are loaded ahead
+    (4, 5, 16, 32, 0),    # two rows a thread (128 heads), one token past the ahead window
+    (8, 3, 16, 32, 1),    # four rows a thread (256 heads), q and k at an odd element
+    (3, 7, 4, 16, 0),     # one row a thread, four value heads per key head
+    (2, 8, 4, 4, 3),      # whole turns of the ahead window, one value head per key head
+    (33, 2, 2, 8, 0),     # four rows a thread (264 heads), a part-filled last run per XCD
+])
+def test_recurrent_rows_per_thread_and_remainders(gpu, B, T, Hk, Hv, off):
+    """The rows-per-thread rule and the token loop's remainders, with q and k
+    off elements (2 bytes each) past an aligned address; a bad slot among the
+    sequences leaves its output and every state untouched."""
+    import torch
+    say("gdn_recurrent", f"B={B} T={T} Hk={Hk} Hv={Hv} off={off}")
+    rng = np.random.default_rng(210 + B + T)
+    inp = gen_recurrent_inputs(rng, B, T, Hk, Hv)
+    pool = _pool(1, B + 2, Hk, Hv)
+    slots = rng.choice(B + 2, B, replace=False).astype(np.int32)
+    pool.write(0, _ids(slots), dev(inp["state"]), None)
+
+    def shifted(a):
+        n = a.size
+        buf = torch.zeros(n + off, dtype=torch.int16, device=gpu)
+        buf[off:] = dev(a).reshape(-1)
+        return buf[off:].view(a.shape)
+
+    q, k = shifted(inp["q"]), shifted(inp["k"])
+    y = torch.zeros((B, T, Hv, DV), dtype=torch.int16, device=gpu)
+    pool.recurrent(0, _ids(slots), q, k, dev(inp["v"]), dev(inp["g"]), dev(inp["beta"]), y)
+    got_s = torch.empty((B, Hv, DV, DK), dtype=torch.float32, device=gpu)
+    pool.read(0, _ids(slots), got_s, None)
+    yr, sr = O.recurrent(inp["q"], inp["k"], inp["v"], inp["g"], inp["beta"], inp["state"])
+    yo = O.bf16_to_f32(yr)
+    dy = np.abs(O.bf16_to_f32(host(y)) - yo)
+    assert np.all(dy <= 2.0 ** -7 * np.abs(yo) + 1e-5 * np.abs(yo).max())
+    assert rel_l2(host(got_s), sr) < 1e-5
+    assert pool.check() == 0
+    bad = slots.copy()
+    bad[0] = B + 2
+    y.fill_(-1)
+    pool.recurrent(0, _ids(bad[:1]), q[:1], k[:1], dev(inp["v"][:1]), dev(inp["g"][:1]),
+                   dev(inp["beta"][:1]), y[:1])
+    again = torch.empty_like(got_s)
+    pool.read(0, _ids(slots), again, None)
+    torch.cuda.synchronize()
+    assert torch.equal(again, got_s) and bool((y[:1] == -1).all())
+    assert pool.check() == 1
+    pool.close()
+
+
 def test_decode_fused_matches_oracle_config0(gpu):
     """One fused decode step, single layer, B=1 (conv state drawn [8192,3]
     channel-major and transposed into the pool's [3,8192] rows)."""
