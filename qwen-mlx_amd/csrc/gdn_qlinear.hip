@@ -169,8 +169,8 @@ __global__ __launch_bounds__(256) void qlinear_xsum_kernel(const uint16_t* __res
   *reinterpret_cast<uint32_t*>(dst + 128 * G) = lo;
 }
 
-// 64 x 128 tiles of four waves in a row, every wave with all 64 rows and two
-// 16-column fragments (the weight fragment is the MFMA A operand: 16 n x 32 k,
+// 16 MW x 128 tiles (MW = 4 but for small batches on very wide layers) of four
+// waves in a row, every wave with all rows and two 16-column fragments (the weight fragment is the MFMA A operand: 16 n x 32 k,
 // the activations the B operand, so a lane ends with four consecutive n of one
 // row m). Takes prefill shapes (M > 64) and, at decode sizes, very wide layers
 // (lm_head). Per stage of 128 k:
@@ -211,15 +211,16 @@ __global__ __launch_bounds__(256) void qlinear_xsum_kernel(const uint16_t* __res
 // 64-column waves (64 x 256 tiles, two waves per SIMD) took 871 and 304 us
 // there but 219 against 199 at M = 3688, where fewer tiles leave a last round
 // half empty.
-template <int KT, int XS>
+template <int MW, int KT, int XS>
 __global__ __launch_bounds__(256)
-    __attribute__((amdgpu_waves_per_eu(KT > 8 && XS == 1 ? 2 : 3, KT > 8 && XS == 1 ? 2 : 3))) void
+    __attribute__((amdgpu_waves_per_eu(MW < 4 ? 4 : KT > 8 && XS == 1 ? 2 : 3,
+                                       MW < 4 ? 4 : KT > 8 && XS == 1 ? 2 : 3))) void
     qlinear_tile_kernel(
     const uint16_t* __restrict__ x, int64_t xs, int M, int K, const uint16_t* __restrict__ wp,
     const uint16_t* __restrict__ sp, const uint16_t* __restrict__ bias,
     const uint16_t* __restrict__ nsc, int N, int Npad, uint16_t* __restrict__ y, int64_t ys,
     const uint16_t* __restrict__ xsg, int Ps, float* __restrict__ part) {
-  constexpr int MW = 4, NW = 2, MT = 64;
+  constexpr int NW = 2, MT = 16 * MW;
   constexpr int XROW = kStageK * 2;  // bytes per staged x row
   constexpr int GMAX = 4 * KT, GJ = GMAX / 32;
   static_assert(GMAX % 32 == 0, "whole 32-group chunks");
@@ -255,7 +256,7 @@ __global__ __launch_bounds__(256)
   __amdgpu_buffer_rsrc_t xrs[4];
   int xvo[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
+  for (int j = 0; j < MW; ++j) {
     const int rb = 4 * (wave + 4 * j), r0 = min(m0 + rb, M - 1);
     const int dr = min(m0 + rb + (lane >> 4), M - 1) - r0;
     xrs[j] = __builtin_amdgcn_make_buffer_rsrc((void*)(x + (int64_t)r0 * xs), (short)0, -1, 0x00020000);
@@ -272,7 +273,7 @@ __global__ __launch_bounds__(256)
     const int p = pofs + ps;
     uint8_t* const xd = S ? xl1 : xl0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < MW; ++j)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           xrs[j], (void __attribute__((address_space(3)))*)(xd + 4 * (wave + 4 * j) * XROW), 16,
           xvo[j], p * XROW, 0, 0);
@@ -300,15 +301,34 @@ __global__ __launch_bounds__(256)
       for (int jb = 0; jb < GJ; ++jb) corr1(i, jb, Ab[i][jb], As[i][jb]);
   };
 
-  if constexpr (XS == 1) {  // the caller's split sums, 3 x 64 rows x G bf16, in 1 KiB copies
+  // XS == 1: the caller's split sums into LDS, [3][MT][G]. All 64 rows are
+  // contiguous per part and go by 1 KiB DMA copies; fewer rows go through
+  // registers (their parts may be smaller than a copy).
+  constexpr int SJ = XS == 1 && MW < 4 ? (3 * MT * GMAX / 8 + 255) / 256 : 1;
+  u32x4 sv[SJ];
+  if constexpr (XS == 1 && MW == 4) {
     const __amdgpu_buffer_rsrc_t grs = __builtin_amdgcn_make_buffer_rsrc(
         (void*)xsg, (short)0, 3 * MT * G * 2, 0x00020000);
     for (int c = wave; c < (3 * MT * G * 2 + 1023) / 1024; c += 4)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(
           grs, (void __attribute__((address_space(3)))*)(sxb + 1024 * c), 16, 1024 * c + 16 * lane,
           0, 0, 0);
+  } else if constexpr (XS == 1) {
+#pragma unroll
+    for (int j = 0; j < SJ; ++j) {
+      const int e = tid + 256 * j, per = MT * G / 8, k = min(e / per, 2);
+      sv[j] = *reinterpret_cast<const u32x4*>(xsg + (int64_t)k * 64 * G +
+                                              8 * min(e - k * per, per - 1));
+    }
   }
   batch(0, std::integral_constant<int, 0>{});
+  if constexpr (XS == 1 && MW < 4) {
+#pragma unroll
+    for (int j = 0; j < SJ; ++j)
+      if (tid + 256 * j < 3 * MT * G / 8)
+        *reinterpret_cast<u32x4*>(sxb + 16 * (tid + 256 * j)) = sv[j];
+    wait_lgkm0();
+  }
   wait_vm<0>();
   __builtin_amdgcn_s_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup", "global");
@@ -409,7 +429,7 @@ __global__ __launch_bounds__(256)
     const int k0 = KT - Ps / 2;
 #pragma unroll
     for (int k = 0; k < KT; ++k)
-      if (k >= k0) sx[(4 * (k - k0) + c4) * MT + wave * 16 + r16] = pk[k];
+      if (k >= k0 && (MW == 4 || wave < MW)) sx[(4 * (k - k0) + c4) * MT + wave * 16 + r16] = pk[k];
   }
   lds_barrier();
 
@@ -419,11 +439,12 @@ __global__ __launch_bounds__(256)
     const bool gin = 32 * jb + 8 * c4 < G;
     if constexpr (XS != 0) {
       const uint16_t* const xsl =
-          XS == 1 ? reinterpret_cast<const uint16_t*>(sxb) : xsg + (int64_t)tm * 3 * MT * G;
+          XS == 1 ? reinterpret_cast<const uint16_t*>(sxb) : xsg + (int64_t)tm * 3 * 64 * G;
+      const int part_rows = XS == 1 ? MT : 64;
       const int o = row * G + (gin ? 32 * jb + 8 * c4 : 0);
       hi = *reinterpret_cast<const u32x4*>(xsl + o);
-      mid = *reinterpret_cast<const u32x4*>(xsl + MT * G + o);
-      lo = *reinterpret_cast<const u32x4*>(xsl + 2 * MT * G + o);
+      mid = *reinterpret_cast<const u32x4*>(xsl + part_rows * G + o);
+      lo = *reinterpret_cast<const u32x4*>(xsl + 2 * part_rows * G + o);
       if (!gin) hi = mid = lo = (u32x4){0u, 0u, 0u, 0u};
     } else {
       const float* const sx = reinterpret_cast<const float*>(sxb);
@@ -517,12 +538,13 @@ __global__ __launch_bounds__(256) void qlinear_tile_sum_kernel(const float* __re
   *reinterpret_cast<u32x2*>(y + (int64_t)m * ys + n) = (u32x2){f2bf2(t[0], t[1]), f2bf2(t[2], t[3])};
 }
 
-// Decode shapes (M <= 64). A work-group owns 64 columns (four 16-wide
+// Decode shapes (M <= 64), 16 MU rows. A work-group owns 64 columns (four 16-wide
 // fragments) and the K slice of NW * SPW stages starting at stage
 // NW * SPW * blockIdx.y; wave w takes SPW stages of it and computes partial
-// sums of all 64 x 64 outputs of its stages. The NW partial tiles are added
-// through LDS at the end in wave order, each wave finishing 16 / NW of the
-// sixteen 16 x 16 tiles (correction and store).
+// sums of all 16 MU x 64 outputs of its stages. The NW partial tiles are added
+// through LDS at the end in wave order, each wave finishing its share of the
+// 4 MU tiles of 16 x 16 (correction and store). A row's sums do not depend on
+// MU: a small batch's rows have the bits they have in a full one.
 //
 // Roles: x is the MFMA A operand and the weights the B operand, so a lane
 // holds D[m][n] for four rows m = 16u + 4c + i and one column n = r16 of the
@@ -552,7 +574,7 @@ __global__ __launch_bounds__(256) void qlinear_tile_sum_kernel(const float* __re
 //
 // With XS the group sums come split from the caller (xsg [3][64][K/64], hi,
 // mid, lo: launch_add_norm's), one K slice only: no X_g products, no split.
-template <int NW, int SPW, bool XS>
+template <int NW, int SPW, int MU, bool XS>
 __global__ __launch_bounds__(64 * NW) void qlinear_decode_kernel(
     const uint16_t* __restrict__ x, int64_t xs, int M, int K, const u32x4* __restrict__ wp,
     const uint16_t* __restrict__ sp, const uint16_t* __restrict__ bias,
@@ -561,15 +583,18 @@ __global__ __launch_bounds__(64 * NW) void qlinear_decode_kernel(
   constexpr int G = 2 * NW * SPW;  // groups of the slice
   constexpr int NG = 2 * SPW;      // groups of a wave
   constexpr int GJ = (G + 31) / 32;
-  constexpr int TPW = 16 / NW;     // tiles each wave finishes
+  constexpr int MT = 16 * MU;      // rows
+  constexpr int NT = 4 * MU;       // 16 x 16 tiles; a wave finishes TPW of them
+  constexpr int TPW = NT < NW ? 1 : NT / NW;
+  constexpr int XL = 2 * MU;       // copies of 8 rows per x group
   constexpr int XR = 32 * GJ + 8;  // bf16 per row of the split X_g arrays (16 B pad)
-  static_assert(NW == 4 || NW == 8, "16 tiles over the waves");
+  static_assert((NW == 4 || NW == 8) && TPW <= MU, "a wave's tiles share a fragment");
   // Per wave two x buffers of one group each (64 rows x 128 B, chunk-swizzled);
   // after the loop the wave's partial tiles (tiles 0-7 in xb0, 8-15 in xb1).
-  __shared__ __align__(16) uint8_t xb0[NW][8192];
-  __shared__ __align__(16) uint8_t xb1[NW][8192];
-  __shared__ __align__(16) float sx[G * 64];          // X_g[m] at sx[g * 64 + m]
-  __shared__ __align__(16) uint16_t xsp[3][64 * XR];  // X_g = hi + mid + lo, [m][g] bf16
+  __shared__ __align__(16) uint8_t xb0[NW][1024 * XL];
+  __shared__ __align__(16) uint8_t xb1[NW][1024 * XL];
+  __shared__ __align__(16) float sx[G * MT];          // X_g[m] at sx[g * MT + m]
+  __shared__ __align__(16) uint16_t xsp[3][MT * XR];  // X_g = hi + mid + lo, [m][g] bf16
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -591,7 +616,7 @@ __global__ __launch_bounds__(64 * NW) void qlinear_decode_kernel(
   auto copy_x = [&](int q, int bq) {
     uint8_t* const sb = bq ? xb1[w] : xb0[w];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < XL; ++i) {
       const int r = 8 * i + drow;
       const int c = (lane & 7) ^ ((4 * i + (drow >> 1)) & 7);
       const int voff = (int)((r * xs + 128 * p0 + 64 * q + 8 * c) * 2);
@@ -621,7 +646,7 @@ __global__ __launch_bounds__(64 * NW) void qlinear_decode_kernel(
       sr[s][f] = __builtin_nontemporal_load(ssrc + (int64_t)f * P * 16 + s * 16);
     }
   // correction operands of the fragment this wave finishes (groups beyond the slice: zero)
-  const int fo = (w * TPW) >> 2;
+  const int fo = (w * TPW) / MU & 3;
   u32x4 Ab[GJ], As[GJ];
 #pragma unroll
   for (int j = 0; j < GJ; ++j) {
@@ -636,7 +661,7 @@ __global__ __launch_bounds__(64 * NW) void qlinear_decode_kernel(
   if constexpr (XS) {
 #pragma unroll
     for (int i = 0; i < TPW; ++i) {
-      const int u = (w * TPW + i) & 3;
+      const int u = (w * TPW + i) % MU;
 #pragma unroll
       for (int j = 0; j < GJ; ++j) {
         const bool gin = 32 * j + 8 * c4 < G;
@@ -652,19 +677,19 @@ __global__ __launch_bounds__(64 * NW) void qlinear_decode_kernel(
   __builtin_amdgcn_sched_barrier(0);
 
   // T[f][u]: D[m][n] for m = 16u + 4c4 + i, n = 16(fb+f) + r16
-  f32x4 T[4][4];
+  f32x4 T[4][MU];
 #pragma unroll
   for (int f = 0; f < 4; ++f)
 #pragma unroll
-    for (int u = 0; u < 4; ++u) T[f][u] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int u = 0; u < MU; ++u) T[f][u] = (f32x4){0.f, 0.f, 0.f, 0.f};
   const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};
   const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
   uint32_t nib = 0x000F000Fu;
   asm volatile("" : "+v"(nib));
   // sel1[u]: the A operand with ones in rows 4u..4u+3 (lane r16 supplies row r16)
-  u32x4 sel1[4];
+  u32x4 sel1[MU];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) sel1[u] = (r16 >> 2) == u ? ones : (u32x4){0u, 0u, 0u, 0u};
+  for (int u = 0; u < MU; ++u) sel1[u] = (r16 >> 2) == u ? ones : (u32x4){0u, 0u, 0u, 0u};
   float xgv[NG];
   constexpr int WS = 8 * SPW + 2 * GJ + (XS ? 3 * TPW * GJ : 0);  // weight, scale, correction loads
 
@@ -672,19 +697,19 @@ __global__ __launch_bounds__(64 * NW) void qlinear_decode_kernel(
   for (int q = 0; q < NG; ++q) {
     const int b = q & 1, s = q >> 1, gl = q & 1;
     // x of group q in LDS: the vector-memory ops issued after its copy may be pending
-    if (q == 0) wait_vm<(NG > 1 ? 8 : 0) + WS>();
-    else if (q == 1) wait_vm<WS + (NG > 2 ? 8 : 0)>();
-    else if (q + 1 < NG) wait_vm<8>();
+    if (q == 0) wait_vm<(NG > 1 ? XL : 0) + WS>();
+    else if (q == 1) wait_vm<WS + (NG > 2 ? XL : 0)>();
+    else if (q + 1 < NG) wait_vm<XL>();
     else wait_vm<0>();
-    u32x4 X[2][4];
+    u32x4 X[2][MU];
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int u = 0; u < 4; ++u) X[j][u] = x_chunk(b, 16 * u + r16, 4 * j + c4);
+      for (int u = 0; u < MU; ++u) X[j][u] = x_chunk(b, 16 * u + r16, 4 * j + c4);
     if constexpr (!XS) {  // D[n][m] += X_g[16u + m] for n in 4u..4u+3: lane (r16, c4) gets X_g[16 c4 + r16]
       f32x4 xg = zero;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < MU; ++u) {
         xg = mfma(sel1[u], X[0][u], xg);
         xg = mfma(sel1[u], X[1][u], xg);
       }
@@ -695,7 +720,7 @@ __global__ __launch_bounds__(64 * NW) void qlinear_decode_kernel(
       const u32x4 A0 = unpack_w(wr[s][f][2 * gl], nib), A1 = unpack_w(wr[s][f][2 * gl + 1], nib);
       const float sc = gl ? bf_hi(sr[s][f]) : bf_lo(sr[s][f]);
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < MU; ++u) {
         f32x4 a = mfma(X[0][u], A0, zero);
         a = mfma(X[1][u], A1, a);
 #pragma unroll
@@ -711,26 +736,27 @@ __global__ __launch_bounds__(64 * NW) void qlinear_decode_kernel(
 
   if constexpr (!XS) {
 #pragma unroll
-    for (int q = 0; q < NG; ++q) sx[(2 * w * SPW + q) * 64 + 16 * c4 + r16] = xgv[q];
+    for (int q = 0; q < NG; ++q)
+      if (MU == 4 || c4 < MU) sx[(2 * w * SPW + q) * MT + 16 * c4 + r16] = xgv[q];
   }
   // partial tiles into the wave's own buffers (all its copies have landed and been read)
 #pragma unroll
   for (int f = 0; f < 4; ++f)
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int t = 4 * f + u;
-      reinterpret_cast<f32x4*>(t < 8 ? xb0[w] : xb1[w])[(t & 7) * 64 + lane] = T[f][u];
+    for (int u = 0; u < MU; ++u) {
+      const int t = MU * f + u;
+      reinterpret_cast<f32x4*>(t < XL ? xb0[w] : xb1[w])[(t & (XL - 1)) * 64 + lane] = T[f][u];
     }
   lds_barrier();
 
   // X_g split once per work-group: thread -> row m, four groups
-  for (int idx = tid; !XS && idx < 64 * 8 * GJ; idx += 64 * NW) {
-    const int m = idx & 63, g0 = 4 * (idx >> 6);
+  for (int idx = tid; !XS && idx < MT * 8 * GJ; idx += 64 * NW) {
+    const int m = idx & (MT - 1), g0 = 4 * (idx / MT);
     uint32_t h2[2], m2[2], l2[2];
 #pragma unroll
     for (int e = 0; e < 4; e += 2) {
-      const float v0 = g0 + e < G ? sx[(g0 + e) * 64 + m] : 0.f;
-      const float v1 = g0 + e + 1 < G ? sx[(g0 + e + 1) * 64 + m] : 0.f;
+      const float v0 = g0 + e < G ? sx[(g0 + e) * MT + m] : 0.f;
+      const float v1 = g0 + e + 1 < G ? sx[(g0 + e + 1) * MT + m] : 0.f;
       const uint32_t h = f2bf2(v0, v1);
       const float q0 = v0 - bf_lo(h), q1 = v1 - bf_hi(h);
       const uint32_t md = f2bf2(q0, q1);
@@ -743,15 +769,16 @@ __global__ __launch_bounds__(64 * NW) void qlinear_decode_kernel(
     *reinterpret_cast<u32x2*>(&xsp[2][m * XR + g0]) = (u32x2){l2[0], l2[1]};
   }
   if constexpr (!XS) lds_barrier();
+  if (NT < NW && w >= NT) return;
 
   const int n = (fb + fo) * 16 + r16;
 #pragma unroll
   for (int i = 0; i < TPW; ++i) {
-    const int t = w * TPW + i, u = t & 3;
-    f32x4 acc = reinterpret_cast<const f32x4*>(t < 8 ? xb0[0] : xb1[0])[(t & 7) * 64 + lane];
+    const int t = w * TPW + i, u = t % MU;
+    f32x4 acc = reinterpret_cast<const f32x4*>(t < XL ? xb0[0] : xb1[0])[(t & (XL - 1)) * 64 + lane];
 #pragma unroll
     for (int v = 1; v < NW; ++v)
-      acc += reinterpret_cast<const f32x4*>(t < 8 ? xb0[v] : xb1[v])[(t & 7) * 64 + lane];
+      acc += reinterpret_cast<const f32x4*>(t < XL ? xb0[v] : xb1[v])[(t & (XL - 1)) * 64 + lane];
     // sum_g (b_g - 128 s_g) X_g, X_g of rows 16u + r16 as the A operand
 #pragma unroll
     for (int jb = 0; jb < GJ; ++jb) {
@@ -797,11 +824,11 @@ __global__ __launch_bounds__(256) void qlinear_sum_kernel(const float* __restric
   *reinterpret_cast<u32x2*>(y + (int64_t)m * ys + n) = (u32x2){f2bf2(t[0], t[1]), f2bf2(t[2], t[3])};
 }
 
-template <int KT, int XS>
+template <int MW, int KT, int XS>
 hipError_t launch_tile(const QLinearArgs& a, int slices = 1) {
-  const int64_t tiles = (int64_t)((a.M + 63) / 64) * (a.Npad / 128);
+  const int64_t tiles = (int64_t)((a.M + 16 * MW - 1) / (16 * MW)) * (a.Npad / 128);
   if (tiles > INT32_MAX) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((qlinear_tile_kernel<KT, XS>), dim3((unsigned)tiles, slices), dim3(256), 0,
+  hipLaunchKernelGGL((qlinear_tile_kernel<MW, KT, XS>), dim3((unsigned)tiles, slices), dim3(256), 0,
                      a.stream, a.x, a.xs, a.M, a.K, reinterpret_cast<const uint16_t*>(a.wp), a.sp,
                      a.bias, a.nsc, a.N, a.Npad, a.y, a.ys, a.xsplit, a.K / 128 / slices,
                      slices > 1 ? a.part : nullptr);
@@ -853,6 +880,12 @@ int qlinear_tile_slices(int K, int64_t tiles) {
 // (qlinear_tile_slices), with the group sums formed once up front where they
 // are many (kSumTiles, kSumColumns).
 //
+// Batches of up to 16 and 32 rows run the same kernels on that many rows: the
+// products, the x copies and the partial tiles shrink with the rows. In graph
+// replays over six layers, M = 16 / 32 / 64: 2048 -> 12,352 6.5 / 7.9 / 10.3 us,
+// 4096 -> 2048 with its slice sum 7.4 / 7.9 / 9.8, 2048 -> 248,320 59 / 67 / 95
+// (the 64-row kernels took 9.9, 9.6 and 87 us at 16 rows).
+//
 // Decode kernel shapes (64 x 12352 x 2048 and 64 x 2048 x 4096, 30 distinct
 // layers): eight waves of two stages for K = 2048 (four waves of four stages,
 // one wave per SIMD, were 20% slower), and for the narrow layer four slices
@@ -878,8 +911,10 @@ hipError_t launch_qlinear(const QLinearArgs& a) {
   if (a.defer) *a.defer = QPartial{};
   if (a.M <= 64 && a.Npad >= kWideDecodeN) {
     const bool xs = a.xsplit != nullptr;
-    if (a.K <= 2048) return xs ? launch_tile<8, 1>(a) : launch_tile<8, 0>(a);
-    return xs ? launch_tile<16, 1>(a) : launch_tile<16, 0>(a);
+    if (a.K > 2048) return xs ? launch_tile<4, 16, 1>(a) : launch_tile<4, 16, 0>(a);
+    if (a.M <= 16) return xs ? launch_tile<1, 8, 1>(a) : launch_tile<1, 8, 0>(a);
+    if (a.M <= 32) return xs ? launch_tile<2, 8, 1>(a) : launch_tile<2, 8, 0>(a);
+    return xs ? launch_tile<4, 8, 1>(a) : launch_tile<4, 8, 0>(a);
   }
   if (a.M <= 64) {
     const int ns = a.part ? qlinear_decode_slices(a.K, a.Npad) : 1;
@@ -887,10 +922,16 @@ hipError_t launch_qlinear(const QLinearArgs& a) {
     if (ksl == 512 || ksl == 1024 || ksl == 2048) {
       const u32x4* wp = reinterpret_cast<const u32x4*>(a.wp);
       const bool xs = a.xsplit != nullptr && ns == 1 && ksl == 2048;
-      auto kern = xs            ? qlinear_decode_kernel<8, 2, true>
-                  : ksl == 2048 ? qlinear_decode_kernel<8, 2, false>
-                  : ksl == 1024 ? qlinear_decode_kernel<8, 1, false>
-                                : qlinear_decode_kernel<4, 1, false>;
+      auto pick = [&](auto mu) {
+        constexpr int MU = decltype(mu)::value;
+        return xs            ? qlinear_decode_kernel<8, 2, MU, true>
+               : ksl == 2048 ? qlinear_decode_kernel<8, 2, MU, false>
+               : ksl == 1024 ? qlinear_decode_kernel<8, 1, MU, false>
+                             : qlinear_decode_kernel<4, 1, MU, false>;
+      };
+      auto kern = a.M <= 16   ? pick(std::integral_constant<int, 1>{})
+                  : a.M <= 32 ? pick(std::integral_constant<int, 2>{})
+                              : pick(std::integral_constant<int, 4>{});
       const int threads = ksl == 512 ? 256 : 512;
       hipLaunchKernelGGL(kern, dim3(a.Npad / 64, ns), dim3(threads), 0, a.stream, a.x, a.xs, a.M,
                          a.K, wp, a.sp, a.bias, a.nsc, a.N, a.y, a.ys, ns > 1 ? a.part : nullptr,
@@ -910,8 +951,8 @@ hipError_t launch_qlinear(const QLinearArgs& a) {
   const int64_t tiles = (int64_t)((a.M + 63) / 64) * (a.Npad / 128);
   const int slices = qlinear_tile_slices(a.K, tiles);
   if (slices > 1 || tiles < kSumTiles || a.Npad < kSumColumns) {
-    if (a.K / slices <= 2048) return launch_tile<8, 0>(a, slices);
-    return launch_tile<16, 0>(a, slices);
+    if (a.K / slices <= 2048) return launch_tile<4, 8, 0>(a, slices);
+    return launch_tile<4, 16, 0>(a, slices);
   }
   QLinearArgs c = a;
   for (int m = 0; m < a.M; m += kQLinearSumRows) {
@@ -924,7 +965,7 @@ hipError_t launch_qlinear(const QLinearArgs& a) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     c.xsplit = a.xsum;
-    if ((e = launch_tile<8, 2>(c)) != hipSuccess) return e;
+    if ((e = launch_tile<4, 8, 2>(c)) != hipSuccess) return e;
   }
   return hipSuccess;
 }

@@ -112,7 +112,7 @@ def test_qlinear_extreme_values(gpu):
 
 
 @pytest.mark.parametrize("M,K", [(1, 2048), (37, 2048), (64, 2048), (64, 512), (17, 1536),
-                                 (64, 4096)])
+                                 (64, 4096), (16, 512), (16, 1024), (32, 2048)])
 def test_qlinear_wide_decode_columns_sampled(gpu, M, K):
     """Decode-sized call on a layer wide enough (131,088 columns) for the
     64 x 128 tile route that lm_head takes, at K = 2048 (lm_head's) and at
@@ -163,6 +163,33 @@ def test_qlinear_prefill_rows_sampled(gpu):
     rows[-1] = M - 1
     yr, ye, mag = O.qmatmul_w4(x[rows], *_merged(parts))
     _check(host(y)[rows], ye, mag, yr, "qlinear M=16384 sampled")
+    layer.close()
+
+
+@pytest.mark.parametrize("M,K,rows", [
+    (m, k, rows) for m in (15, 16, 17, 32, 33)
+    for k, rows in ((512, [80]), (2048, [8192, 16]), (2048, [1024]), (4096, [144]))])
+def test_qlinear_small_batches_match_full_batch(gpu, M, K, rows):
+    """Decode-sized calls of up to 16, 32 and 64 rows run kernels of that many
+    rows: the oracle's bar, and the same bits as the same rows in a 64-row
+    call, on one-slice and K-sliced layers."""
+    import torch
+    say("gdn_qlinear_forward", f"small batch M={M} K={K} rows={rows}")
+    rng = np.random.default_rng(506 + M + K)
+    parts = _parts(rng, K, rows)
+    N = sum(rows)
+    x = O.f32_to_bf16(rng.standard_normal((64, K)).astype(np.float32))
+    layer = _layer(K, parts)
+    y = torch.full((M, N + 4), -1, dtype=torch.int16, device=gpu)
+    full = torch.empty((64, N), dtype=torch.int16, device=gpu)
+    layer.forward(dev(x[:M]), y)
+    layer.forward(dev(x), full)
+    torch.cuda.synchronize()
+    assert torch.equal(y[:, :N], full[:M]) and bool((y[:, N:] == -1).all())
+    cols = np.sort(rng.choice(N, min(N, 512), replace=False))
+    w, s, b = (a[cols] for a in _merged(parts))
+    yr, ye, mag = O.qmatmul_w4(x[:M], w, s, b)
+    _check(host(y)[:, cols], ye, mag, yr, f"qlinear small batch M={M} K={K}")
     layer.close()
 
 

@@ -54,7 +54,7 @@ def _split3(s):
     return hi, md, lo
 
 
-@pytest.mark.parametrize("M", [1, 37, 64])
+@pytest.mark.parametrize("M", [1, 16, 17, 32, 37, 64])
 def test_norm_group_sums_projection_matches_oracle(gpu, M):
     import torch
 
@@ -133,7 +133,8 @@ def test_add_rms_norm_adds_and_checks(gpu):
         gdn_amd.add_rms_norm(odd, None, dev(w), 1e-6, torch.empty_like(odd))  # hidden % 8
 
 
-@pytest.mark.parametrize("M,K", [(1, 2048), (37, 2048), (64, 2048), (5, 1024), (64, 4096)])
+@pytest.mark.parametrize("M,K", [(1, 2048), (37, 2048), (64, 2048), (5, 1024), (64, 4096),
+                                 (16, 512), (17, 1536), (32, 2048)])
 def test_norm_group_sums_wide_head_matches_oracle(gpu, M, K):
     """The lm_head route with the norm's group sums: 131,088 columns (over the
     131,072 threshold, the last 128-column tile part padding), K = 2048
