@@ -884,7 +884,7 @@ int qlinear_tile_slices(int K, int64_t tiles) {
 // products, the x copies and the partial tiles shrink with the rows. In graph
 // replays over six layers, M = 16 / 32 / 64: 2048 -> 12,352 6.5 / 7.9 / 10.3 us,
 // 4096 -> 2048 with its slice sum 7.4 / 7.9 / 9.8, 2048 -> 248,320 59 / 67 / 95
-// (the 64-row kernels took 9.9, 9.6 and 87 us at 16 rows).
+// (the 64-row kernels took 10.0, 9.1 and 90 us at 16 rows).
 //
 // Decode kernel shapes (64 x 12352 x 2048 and 64 x 2048 x 4096, 30 distinct
 // layers): eight waves of two stages for K = 2048 (four waves of four stages,
