@@ -220,12 +220,13 @@ gdn_status gdn_decode_gated(gdn_pool* pool, int32_t layer, const int32_t* slot_i
  * clamp every bound they read). Uses the chunked (WY form, chunk 64)
  * algorithm; results equal the token-by-token recurrence within f32/bf16
  * rounding. Two schedules give the same bits: one work-group per (sequence,
- * value head), or, for a few long sequences (at most 96 sequence-heads, 1024
- * tokens per sequence on average, 262,144 tokens per call), the chunks'
+ * value head), or, for few sequences (at most 128 sequence-heads and 262,144
+ * tokens per call, 256 tokens per sequence on average, 768 above 96
+ * sequence-heads), the chunks'
  * state-independent blocks formed for all chunks at once and 2 or 4
  * work-groups per (sequence, value head). The environment variable
  * GDN_PREFILL_WAVES = 8 (the first), 4 or 2 (the second) forces one.
- * The second schedule, with at least 8,192 tokens in the call and at most
+ * The second schedule, for one sequence of at least 8,192 tokens and at most
  * half as many work-groups as the device has CUs (one 16,384-token prompt at
  * 32 value heads: 128), runs as a pipeline of 2 to 8 token segments (each
  * twice the one before): the next

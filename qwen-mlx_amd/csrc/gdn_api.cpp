@@ -620,7 +620,7 @@ static gdn_status prefill_common(gdn_pool* pool, int32_t layer, const int32_t* s
   // The split path pipelines its segments over a second stream, except under
   // stream capture and in the no-allocation entry (which makes no objects).
   const int groups = pool->d.num_v_heads * nseq * (waves ? 8 / waves : 1);
-  const int segs = gdn::prefill_pipeline_segments(waves, total_tokens, groups, pool->cus);
+  const int segs = gdn::prefill_pipeline_segments(waves, nseq, total_tokens, groups, pool->cus);
   if (!noalloc && segs > 1) {
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(a.stream, &cs) != hipSuccess) {

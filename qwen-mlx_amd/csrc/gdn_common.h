@@ -276,7 +276,7 @@ int prefill_chunk_waves(int R, int Hk, int nseq, int total_tokens);
 // Segments of a pipelined prefill call on the path `waves` picked, whose
 // chunk kernel has `groups` work-groups, on a device of `cus` CUs (1: one
 // pass, no second stream).
-int prefill_pipeline_segments(int waves, int total_tokens, int groups, int cus);
+int prefill_pipeline_segments(int waves, int nseq, int total_tokens, int groups, int cus);
 size_t prefill_workspace_bytes(int R, int Hk, int total_tokens, int nseq, int waves, bool y_scratch);
 size_t prefill_workspace_reserve_bytes(int R, int Hk, int max_tokens);
 // Fixed per-device workspace of gdn_prefill_varlen_noalloc (gdn_prefill.hip).

@@ -26,10 +26,13 @@ constexpr float kQNormW = 0.0078125f;
 constexpr float kKNormW = 0.08837890625f;
 constexpr float kNormEps = 1e-6f;
 constexpr int kTT = 64;  // tokens per qkv_kernel work-group
-// The split path is taken for prompts of at least kSplitMinTokens tokens on
-// average and calls of at most kSplitMaxTokens tokens (its records take 272
-// bytes per token and value head).
-constexpr int kSplitMinTokens = 1024;
+// The split path is taken for calls of at most kSplitMaxGroups sequence-heads
+// and kSplitMaxTokens tokens (its records take 272 bytes per token and value
+// head) whose prompts hold at least kSplitMinTokens tokens on average, or
+// kSplitMinTokensFull above 96 sequence-heads (see prefill_chunk_waves).
+constexpr int kSplitMinTokens = 256;
+constexpr int kSplitMinTokensFull = 768;
+constexpr int kSplitMaxGroups = 128;
 constexpr int kSplitMaxTokens = 1 << 18;
 constexpr int kRecStride = 17408;  // bytes per chunk record (kRecBytes)
 
@@ -1315,9 +1318,17 @@ __global__ __launch_bounds__(256) void prefill_norm_gate_kernel(
 // Waves per work-group of the chunk kernel for a call: 8 runs the fused
 // chunk kernel alone (one group per (sequence, value head)); 2 or 4 run the
 // split path (prefill_form_kernel, then 8/W groups per (sequence, value
-// head)) where the fused kernel would leave most CUs idle: few sequences of
-// many chunks. The environment variable GDN_PREFILL_WAVES = 2, 4 or 8 forces
-// a path (tests compare the paths with it).
+// head)) where the fused kernel would leave at least half of the CUs idle: up
+// to 128 sequence-heads, one work-group each. A chunk then takes about 3.3 us
+// of the longest prompt's chain against 5.6, and the forming of the blocks is
+// paid up front. Measured per call, fused against split, us: 16/32 heads one
+// prompt of 128 tokens 23.7 / 23.9, 256 33.7 / 30.1, 512 55 / 46; three of 37,
+// 512 and 1,200 118 / 99; four of 512 71.4 / 73.3, of 128, 512, 1,000 and 2,048
+// 193 / 164, of 2,048 226 / 222, of 16,384 1,648 / 1,610; 4/16 heads six of
+// 1,000 109 / 106; 4/4 heads eight of 512 56.5 / 51, of 2,048 183 / 156. Beyond
+// 128 sequence-heads the fused kernel fills the chip: 16/32 heads six of 1,000
+// 140 / 196. The environment variable GDN_PREFILL_WAVES = 2, 4 or 8 forces a
+// path (tests compare the paths with it).
 // The path GDN_PREFILL_WAVES forces (2, 4 or 8), or 0.
 static int forced_chunk_waves() {
   if (const char* v = getenv("GDN_PREFILL_WAVES")) {
@@ -1330,29 +1341,26 @@ static int forced_chunk_waves() {
 int prefill_chunk_waves(int R, int Hk, int nseq, int total_tokens) {
   if (const int f = forced_chunk_waves()) return total_tokens > 0 ? f : 8;
   if (nseq <= 0 || total_tokens <= 0 || total_tokens > kSplitMaxTokens) return 8;
-  if (total_tokens / nseq < kSplitMinTokens) return 8;
-  // measured on 16,384-token prompts (32 value heads): one or two prompts
-  // 1.10 / 1.30 ms split against 1.36 / 1.50 ms fused per call; four prompts
-  // 1.80 ms with 4-wave groups against 1.76 ms fused
-  const int groups = nseq * Hk * R;
-  return groups <= 64 ? 2 : groups <= 96 ? 4 : 8;
+  const int groups = nseq * Hk * R, avg = total_tokens / nseq;
+  if (groups > kSplitMaxGroups || avg < (groups > 96 ? kSplitMinTokensFull : kSplitMinTokens)) return 8;
+  return groups <= 64 ? 2 : 4;
 }
 
 // When the split path's chunk kernel leaves at least half of the CUs idle (its
 // groups, one per CU, number at most half the CUs), a call of at least two
 // segments of kPipeSegmentTokens runs its qkv and form kernels one segment
 // ahead on a second stream, beside the chunk kernel of the previous segment.
-// At 32 value heads that admits one prompt. Pipelining several long prompts
-// loses: segments cut the packed tokens, so a later prompt falls wholly into
+// Only one prompt is pipelined; several lose: segments cut the packed tokens, so a later prompt falls wholly into
 // the last segments and its chain starts only after the first prompt's (two
 // 16,384-token prompts forced into segments: 1.72-1.75 ms per layer at 256
-// 2-wave groups, 1.68-1.72 at 128 4-wave groups, against 1.19 in one pass).
+// 2-wave groups, 1.68-1.72 at 128 4-wave groups, against 1.19 in one pass; at
+// 4/4 heads four of 16,384 2.46 ms against 0.92).
 // GDN_PREFILL_SEGMENTS = n forces n segments (1: one pass) on the split path.
 constexpr int kPipeSegmentTokens = 4096;
 
-int prefill_pipeline_segments(int waves, int total_tokens, int groups, int cus) {
+int prefill_pipeline_segments(int waves, int nseq, int total_tokens, int groups, int cus) {
   if (waves != 2 && waves != 4) return 1;
-  if ((waves != 2 || 2 * (int64_t)groups > cus) && !getenv("GDN_PREFILL_SEGMENTS")) return 1;
+  if ((waves != 2 || nseq > 1 || 2 * (int64_t)groups > cus) && !getenv("GDN_PREFILL_SEGMENTS")) return 1;
   const int tiles = (total_tokens + kTT - 1) / kTT;
   int n = total_tokens / kPipeSegmentTokens;
   if (const char* v = getenv("GDN_PREFILL_SEGMENTS")) n = atoi(v);
@@ -1373,7 +1381,7 @@ size_t prefill_workspace_reserve_bytes(int R, int Hk, int max_tokens) {
     most = std::max(most, prefill_workspace_bytes(R, Hk, max_tokens, std::max(max_tokens, 1), f,
                                                   true));
   if (max_tokens > kSplitMaxTokens) max_tokens = kSplitMaxTokens;
-  for (int nseq = 1; nseq * Hk * R <= 96 && nseq <= max_tokens; ++nseq)
+  for (int nseq = 1; nseq * Hk * R <= kSplitMaxGroups && nseq <= max_tokens; ++nseq)
     most = std::max(most, prefill_workspace_bytes(R, Hk, max_tokens, nseq, 2, true));
   return most;
 }

@@ -383,6 +383,59 @@ def test_prefill_pipelined_segments_match_one_pass(gpu, prefill_waves, prefill_s
             assert np.array_equal(a, b), f"waves, segments = {key}: {what} differs from the fused path"
 
 
+@pytest.mark.parametrize("Hk,Hv,lens", [
+    (16, 32, [255]),                      # one token short of the split schedule
+    (16, 32, [256]),                      # its shortest prompt
+    (16, 32, [767, 0, 1]),                # 96 sequence-heads, average 256
+    (16, 32, [5, 17, 900, 2150]),         # 128 sequence-heads, average 768
+    (16, 32, [5, 17, 900, 2149]),         # and one token below
+    (16, 32, [300, 1, 700, 900, 64]),     # 160 sequence-heads: fused
+    (4, 16, [1024, 3, 700, 129, 512, 64, 40, 3700]),  # 128 sequence-heads, average 771
+    (4, 4, [5000, 1, 3500]),              # 8,192 tokens and few groups, but not one prompt
+])
+def test_prefill_schedule_rule_edges_match_fused(gpu, prefill_waves, Hk, Hv, lens):
+    """The library's own choice of schedule at the edges of its rule against
+    the fused chunk kernel forced: y, gated out, state and conv window are the
+    same bits, and two calls in a row (the second from the first's states, on
+    a workspace that already exists) too."""
+    import gdn_amd
+    import torch
+    say("gdn_prefill_varlen schedule rule", f"lens={lens} Hk={Hk} Hv={Hv}")
+    rng = np.random.default_rng(640 + Hk + len(lens))
+    n, T, D = len(lens), sum(lens), conv_dim(Hk, Hv)
+    p = gen_layer_params(rng, Hk, Hv)
+    st0, cs0 = gen_states(rng, n, Hk, Hv, state_std=0.05)
+    mixed, ab = gen_tokens(rng, T, Hk, Hv)
+    qkvz = np.zeros((T, D + Hv * DV), np.uint16)
+    qkvz[:, :D] = mixed
+    qkvz[:, D:] = O.f32_to_bf16(rng.standard_normal((T, Hv * DV)).astype(np.float32))
+    norm_w = dev(O.f32_to_bf16((1.0 + 0.1 * rng.standard_normal(DV)).astype(np.float32)))
+    cu = dev(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32))
+    slots = rng.permutation(n + 2)[:n].astype(np.int32)
+    ids = _ids(slots)
+    args = (dev(ab), dev(p["A_log"]), dev(p["dt_bias"]), dev(p["conv_w"]))
+    md, qd = dev(mixed), dev(qkvz)
+    res = {}
+    for w in (8, 0):
+        prefill_waves(w)
+        got = []
+        for gated in (False, True):
+            pool = gdn_amd.Pool(1, n + 2, Hk, Hv)
+            pool.write(0, ids, dev(st0), dev(cs0))
+            for _ in range(2):
+                y = torch.zeros((T, Hv, DV), dtype=torch.int16, device=gpu)
+                if gated:
+                    pool.prefill_gated(0, ids, cu, T, qd, *args, norm_w, 1e-6, y)
+                else:
+                    pool.prefill(0, ids, cu, T, md, *args, y)
+                got += [host(y), *_read(pool, 0, slots, gpu)]
+            assert pool.check() == 0
+            pool.close()
+        res[w] = got
+    for i, (a, b) in enumerate(zip(res[8], res[0])):
+        assert np.array_equal(a, b), f"output {i} differs from the fused schedule"
+
+
 def test_prefill_one_long_prompt_pipelined_matches_one_pass(gpu, prefill_segments):
     """One 16,384-token prompt takes the split path in 4 segments by default;
     its y, state and conv window equal the one-pass call's bit for bit, and a
