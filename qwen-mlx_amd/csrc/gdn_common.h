@@ -288,6 +288,7 @@ hipError_t launch_prefill(const PrefillArgs& a);
 struct AttnArgs {
   int T, Hq, Hkv, P, max_pages, rot_dim;
   int NC, kpw;             // chunks of work in the step, chunks per worker
+  int max_chunks;          // of the longest segment
   bool stream_keys;        // each block read about once (non-temporal loads)
   float eps, log2_base;
   const uint16_t* q_full;  // [T, qs]: per query head 256 query then 256 gate values
@@ -303,6 +304,8 @@ struct AttnArgs {
   const int32_t* grp;      // [groups][4]: first token, tokens, first position, slot
   const int32_t* seg;      // [groups * Hkv][4]: first chunk, chunks, -, -
   const int32_t* wseg;     // [P]: segment of each worker's first chunk
+  const int32_t* tiles;    // [NT][4]: prompt tiles: first token, tokens, first position, slot
+  int NT;
   int32_t* ptab;           // [num_slots][max_pages] page table
   uint16_t* pages;         // this layer's pages [num_pages][2][Hkv][16384]
   uint16_t* out;           // [T, os]: Hq x 256 gated attention rows
@@ -311,7 +314,8 @@ struct AttnArgs {
   hipStream_t stream;
 };
 size_t attn_workspace_bytes(int T, int Hq, int64_t chunks);
-int attn_chunk_blocks();  // 16-key blocks per chunk
+int attn_chunk_keys();  // keys per chunk (one partial)
+int attn_block_keys();  // keys per block
 hipError_t launch_attn(const AttnArgs& a);
 // A sequence's cached rows of one layer into [Hkv][len][256] K and V arrays.
 hipError_t launch_kv_gather(const uint16_t* pages, const int32_t* prow, int Hkv, int64_t len,

@@ -12,14 +12,16 @@
 // for all layers), then each attention layer runs gdn_attn_forward on the
 // same packed tokens.
 //
-// The schedule: the step's tokens form groups of up to 16 / G consecutive
-// tokens of one sequence (G query heads per kv head: a group's (token, head)
-// pairs fill the 16 columns of an MFMA tile); each (group, kv head) segment
-// is its keys, cut into chunks of 384 keys at fixed points. All segments'
-// chunks, in order, go to P one-wave workers in equal runs of kpw, P up to
-// max_workers (default below). Every chunk writes one partial and the
-// combine kernel merges a segment's partials in order, so a token's result
-// does not depend on the rest of the step.
+// The schedule. Prompts whose tiles fill the chip run as tiles of 128 / G tokens,
+// each through all its keys in one work-group (see use_tiles). The other tokens
+// form groups of up to 16 / G consecutive tokens of one sequence (G query heads
+// per kv head: a group's (token, head) pairs fill the 16 columns of an MFMA
+// tile); each (group, kv head) segment is its keys, cut into chunks of 384 keys
+// at fixed points. All segments' chunks, in order, go to P one-wave workers in
+// equal runs of kpw, P up to max_workers (default below). Every chunk writes one
+// partial and the combine kernel merges a segment's partials in order. Tiles
+// merge the same chunks the same way, so a token's result does not depend on
+// the rest of the step or on the route.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -58,7 +60,22 @@ constexpr int kStreamWorkers = 1536;  // equal runs of chunks: 768 .. 1536 worke
 constexpr int kReuseWorkers = 2048;
 
 // int32 words of the step metadata for up to T tokens and P workers
-size_t meta_words(int T, int Hkv, int P) { return (size_t)T * (5 + 4 + 4 * (size_t)Hkv) + P; }
+// (tiles: four words for every 16 tokens or more, and one part-filled per sequence of
+// at least kTileMinTokens)
+size_t meta_words(int T, int Hkv, int P) { return (size_t)T * (5 + 4 + 4 * (size_t)Hkv) + P + T + 4; }
+
+// A sequence with at least this many new tokens can run as tiles.
+constexpr int kTileMinTokens = 16;
+
+// Tiles or chunks for the step's prompts: `work` 32-key blocks over all their
+// tiles, `longest` of the longest one. A tile block takes about 2.07 us on its CU
+// and a tile's blocks run one after the other; the chunk route takes about 19.5
+// ns per tile block with the whole chip at work on it (16/2 heads, measured on
+// 1,024 to 4,096 new tokens behind 0 to 4,096 cached ones). So tiles win once
+// their work passes 100 of the longest: 2,048 tokens 157 us against 185, behind
+// 2,048 cached ones 281 against 490, 4,096 tokens 322 against 710; 512 tokens
+// behind 4,096 stay on chunks, 145 against 304.
+bool use_tiles(int64_t work, int64_t longest) { return work > 100 * longest; }
 
 int max_workers(const gdn_kv_desc& d) { return d.max_workers > 0 ? d.max_workers : kReuseWorkers; }
 
@@ -90,7 +107,7 @@ struct gdn_kv {
   void* workspace = nullptr;
   size_t ws_bytes = 0;
   // the planned step
-  int T = 0, NG = 0, P = 0, NC = 0, kpw = 0;
+  int T = 0, NG = 0, P = 0, NC = 0, kpw = 0, NT = 0, max_chunks = 0;
   bool stream_keys = false;
   bool planned = false;
 };
@@ -154,15 +171,15 @@ gdn_status gdn_kv_create(const gdn_kv_desc* desc, gdn_kv** out) {
   }
   // The attention workspace of any decode step (one token per sequence),
   // sized once: n <= min(max_step_tokens, num_slots) sequences, each
-  // segment's keys cut into chunks of C blocks. Sequences hold distinct
-  // pages, so their blocks add up to at most 4 per page in the cache plus
-  // one partial block each: chunks <= Hkv (n + (4 num_pages + 2 n) / C + 2).
+  // segment's keys cut into chunks of C keys. Sequences hold distinct pages,
+  // so their keys add up to at most 64 per page in the cache: chunks <=
+  // Hkv (n + 64 num_pages / C + 2).
   // A step with prompts (several tokens of one sequence, each group of them
   // reading the shared prefix) can need more and then grows it.
   {
     const int64_t n = d.max_step_tokens < d.num_slots ? d.max_step_tokens : d.num_slots;
     const int64_t chunks =
-        (int64_t)d.num_kv_heads * (n + (4 * (int64_t)d.num_pages + 2 * n) / gdn::attn_chunk_blocks() + 2);
+        (int64_t)d.num_kv_heads * (n + (int64_t)kPageTokens * d.num_pages / gdn::attn_chunk_keys() + 2);
     const size_t ws = gdn::attn_workspace_bytes((int)n, d.num_q_heads, chunks);
     if (hipMalloc(&kv->workspace, ws) != hipSuccess) {
       (void)hipGetLastError();
@@ -256,27 +273,48 @@ gdn_status gdn_kv_step(gdn_kv* kv, int32_t n, const int32_t* slots, const int32_
   struct Group {
     int32_t t0, ntok, pos0, slot;
   };
-  std::vector<Group> groups;
+  std::vector<Group> groups, tiles;
+  const int BK = gdn::attn_block_keys();
+  const int tpt = 128 / G;  // tokens per tile
   {
+    int64_t work = 0, longest = 0;
+    for (int i = 0; i < n; ++i) {
+      if (ntok[i] < kTileMinTokens) continue;
+      for (int32_t k = 0; k < ntok[i]; k += tpt) {
+        const int64_t last = kv->len[slots[i]] + std::min(k + tpt, ntok[i]);
+        const int64_t nb = (last + BK - 1) / BK;
+        work += nb * Hkv;
+        longest = std::max(longest, nb);
+      }
+    }
+    const bool tiled = use_tiles(work, longest);
     int32_t t0 = 0;
     for (int i = 0; i < n; ++i) {
-      for (int32_t k = 0; k < ntok[i]; k += tpg) {
-        const int32_t nt = ntok[i] - k < tpg ? ntok[i] - k : tpg;
-        groups.push_back({t0 + k, nt, (int32_t)(kv->len[slots[i]] + k), slots[i]});
+      const bool tile = tiled && ntok[i] >= kTileMinTokens;
+      const int32_t step = tile ? tpt : tpg;
+      for (int32_t k = 0; k < ntok[i]; k += step) {
+        const int32_t nt = ntok[i] - k < step ? ntok[i] - k : step;
+        (tile ? tiles : groups).push_back({t0 + k, nt, (int32_t)(kv->len[slots[i]] + k), slots[i]});
       }
       t0 += ntok[i];
     }
+    // longest first: the last tiles to start are short ones
+    std::stable_sort(tiles.begin(), tiles.end(), [](const Group& a, const Group& b) {
+      return a.pos0 + a.ntok > b.pos0 + b.ntok;
+    });
   }
+  const int NT = (int)tiles.size();
   const int NG = (int)groups.size(), NS = NG * Hkv;
-  // each segment's keys in chunks of C 16-key blocks, numbered in segment order
-  const int C = gdn::attn_chunk_blocks();
+  // each segment's keys in chunks of C keys, numbered in segment order
+  const int C = gdn::attn_chunk_keys();
   std::vector<int64_t> cs0(NS + 1);
   cs0[0] = 0;
-  int64_t W = 0, distinct = 0;
+  int64_t W = 0, distinct = 0, max_chunks = 0;
   for (int gi = 0; gi < NG; ++gi) {
-    const int64_t nblk = ((int64_t)groups[gi].pos0 + groups[gi].ntok + 15) / 16;
-    for (int j = 0; j < Hkv; ++j) cs0[gi * Hkv + j + 1] = cs0[gi * Hkv + j] + (nblk + C - 1) / C;
+    const int64_t keys = (int64_t)groups[gi].pos0 + groups[gi].ntok, nblk = (keys + BK - 1) / BK;
+    for (int j = 0; j < Hkv; ++j) cs0[gi * Hkv + j + 1] = cs0[gi * Hkv + j] + (keys + C - 1) / C;
     W += nblk * Hkv;
+    max_chunks = std::max(max_chunks, (keys + C - 1) / C);
     // distinct blocks: each sequence's keys once per kv head (its last group's)
     if (gi + 1 == NG || groups[gi + 1].slot != groups[gi].slot) distinct += nblk * Hkv;
   }
@@ -285,7 +323,8 @@ gdn_status gdn_kv_step(gdn_kv* kv, int32_t n, const int32_t* slots, const int32_
   const bool stream_keys = W < 2 * distinct;
   const int pmax = d.max_workers > 0 ? d.max_workers : (stream_keys ? kStreamWorkers : kReuseWorkers);
   // equal runs of kpw chunks: kpw = ceil(NC / pmax), P = ceil(NC / kpw) <= pmax
-  const int kpw = (int)((NC + pmax - 1) / pmax);
+  // (none when every token is in a tile)
+  const int kpw = std::max(1, (int)((NC + pmax - 1) / pmax));
   const int P = (int)((NC + kpw - 1) / kpw);
   std::vector<int32_t> wseg(P);
   {
@@ -321,6 +360,15 @@ gdn_status gdn_kv_step(gdn_kv* kv, int32_t n, const int32_t* slots, const int32_
   int32_t* m_grp = kv->p_meta + 5 * T;
   int32_t* m_seg = m_grp + 4 * NG;
   int32_t* m_wseg = m_seg + 4 * NS;
+  int32_t* m_tile = m_wseg + P;
+  for (int i = 0; i < NT; ++i) {
+    const Group& g = tiles[i];
+    m_tile[4 * i] = g.t0;
+    m_tile[4 * i + 1] = g.ntok;
+    m_tile[4 * i + 2] = g.pos0;
+    m_tile[4 * i + 3] = g.slot;
+    for (int k = 0; k < g.ntok; ++k) m_tokseg[g.t0 + k] = m_tokseg[T + g.t0 + k] = -1;
+  }
   for (int gi = 0; gi < NG; ++gi) {
     const Group& g = groups[gi];
     m_grp[4 * gi] = g.t0;
@@ -339,7 +387,7 @@ gdn_status gdn_kv_step(gdn_kv* kv, int32_t n, const int32_t* slots, const int32_
     m_seg[4 * sg + 3] = 0;
   }
   for (int ww = 0; ww < P; ++ww) m_wseg[ww] = wseg[ww];
-  const size_t words = (size_t)5 * T + 4 * (size_t)NG + 4 * (size_t)NS + P;
+  const size_t words = (size_t)5 * T + 4 * (size_t)NG + 4 * (size_t)NS + P + 4 * (size_t)NT;
   int64_t t = 0;
   for (int i = 0; i < n; ++i) {
     const int32_t sl = slots[i];
@@ -365,6 +413,8 @@ gdn_status gdn_kv_step(gdn_kv* kv, int32_t n, const int32_t* slots, const int32_
   kv->NG = NG;
   kv->P = P;
   kv->NC = (int)NC;
+  kv->NT = NT;
+  kv->max_chunks = (int)max_chunks;
   kv->kpw = kpw;
   kv->stream_keys = stream_keys;
   kv->planned = true;
@@ -416,6 +466,9 @@ gdn_status gdn_attn_forward(gdn_kv* kv, int32_t layer, const uint16_t* q_full, i
   a.grp = kv->d_meta + 5 * (size_t)kv->T;
   a.seg = a.grp + 4 * (size_t)kv->NG;
   a.wseg = a.seg + 4 * (size_t)kv->NG * d.num_kv_heads;
+  a.tiles = a.wseg + kv->P;
+  a.NT = kv->NT;
+  a.max_chunks = kv->max_chunks;
   a.ptab = kv->ptab;
   a.pages = kv->pages[layer];
   a.out = out;

@@ -184,7 +184,8 @@ hipError_t launch_prefill(const PrefillArgs&) { return hipSuccess; }
 size_t attn_workspace_bytes(int T, int Hq, int64_t chunks) {
   return (size_t)T * Hq * 256 * 2 + (size_t)chunks * 16 * 260 * 4 + 256;
 }
-int attn_chunk_blocks() { return 24; }
+int attn_chunk_keys() { return 384; }
+int attn_block_keys() { return 32; }
 hipError_t launch_attn(const AttnArgs&) { return hipSuccess; }
 hipError_t launch_kv_gather(const uint16_t*, const int32_t*, int, int64_t, uint16_t*, uint16_t*,
                             hipStream_t) {

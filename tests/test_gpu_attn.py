@@ -207,6 +207,68 @@ def test_attention_prompt_split_over_steps_is_bit_identical(gpu):
     kb.close()
 
 
+@pytest.mark.parametrize("Hq,Hkv", [(16, 2), (8, 2)])
+def test_attention_tiles_equal_chunks(gpu, Hq, Hkv):
+    """Ragged prompts (tile edges: 16, 17, 127, 128, 129 tokens; some
+    behind cached tokens) and decode tokens in one step, enough work for the
+    prompt tiles, against each sequence stepped alone, which takes the chunk
+    route: outputs and caches bit-identical, and one sequence against the
+    oracle. The rows are column slices at an odd element of wider arrays."""
+    import torch
+
+    import gdn_amd
+    say("gdn_attn_forward", f"tiles vs chunks Hq={Hq}")
+    rng = np.random.default_rng(1450 + Hq)
+    cached = [0, 0, 33, 400, 0, 383, 0, 64, 0, 1, 0, 385, 70, 5] * (32 // Hq - 1)
+    ntok = [300, 16, 290, 17, 300, 129, 256, 300, 128, 300, 127, 270, 1, 1] * (len(cached) // 14)
+    n = len(ntok)
+    # the step's tiles of 128 / G tokens: their 32-key blocks against the longest's
+    nb = [-(-(c + min(k + 128 * Hkv // Hq, m)) // 32) for c, m in zip(cached, ntok) if m >= 16
+          for k in range(0, m, 128 * Hkv // Hq)]
+    assert sum(nb) * Hkv > 100 * max(nb), "the step would not take the tile route"
+    ka, kb = (gdn_amd.KVCache(1, n, 16 * n, 16, Hq, Hkv, max_step_tokens=8192) for _ in range(2))
+    seqs = _Seqs(rng, Hq, Hkv, 1)
+    w = (dev(seqs.w[0][0]), dev(seqs.w[0][1]))
+
+    def rows(m):
+        hosts = seqs.rows(m)
+        wide = [torch.zeros((m, a.shape[1] + 3), dtype=torch.int16, device=gpu) for a in hosts]
+        for t, a in zip(wide, hosts):
+            t[:, 1:-2] = dev(a)
+        return hosts, [t[:, 1:-2] for t in wide]
+
+    pre = [i for i in range(n) if cached[i]]
+    for kv in (ka, kb):
+        seqs.rng = np.random.default_rng(7)
+        _, (q, k, v) = rows(sum(cached))
+        out = torch.empty((sum(cached), Hq * HD), dtype=torch.int16, device=gpu)
+        kv.step(pre, [cached[i] for i in pre])
+        kv.forward(0, q, k, v, *w, EPS, THETA, ROT, out)
+    T = sum(ntok)
+    hosts, (q, k, v) = rows(T)
+    oa = torch.full((T, Hq * HD + 3), -1, dtype=torch.int16, device=gpu)
+    ob = torch.empty((T, Hq * HD), dtype=torch.int16, device=gpu)
+    ka.step(list(range(n)), ntok)
+    ka.forward(0, q, k, v, *w, EPS, THETA, ROT, oa[:, 1:-2])
+    r0 = 0
+    for s, m in enumerate(ntok):
+        kb.step([s], [m])
+        kb.forward(0, q[r0:r0 + m], k[r0:r0 + m], v[r0:r0 + m], *w, EPS, THETA, ROT, ob[r0:r0 + m])
+        r0 += m
+    torch.cuda.synchronize()
+    assert torch.equal(oa[:, 1:-2], ob)
+    assert bool((oa[:, 0] == -1).all()) and bool((oa[:, -2:] == -1).all())
+    for s in range(n):
+        for x, y in zip(ka.read(0, s), kb.read(0, s)):
+            assert torch.equal(x, y)
+    ref = seqs.oracle(0, 0, *(a[:300] for a in hosts))
+    err = rel_l2(O.bf16_to_f32(host(oa[:300, 1:-2].contiguous())), O.bf16_to_f32(ref))
+    say("tiles vs oracle", f"relL2 {err:.2e}")
+    assert err <= 1e-2
+    ka.close()
+    kb.close()
+
+
 def test_attention_long_context_splits(gpu):
     """A 2,500-token context (three 1,024-key splits) built by prefill steps of
     1,000 and 1,500 tokens, then two decode steps, against the oracle."""
