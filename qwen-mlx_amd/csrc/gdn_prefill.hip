@@ -45,8 +45,10 @@ struct Workspace {
   uint16_t* beta;
   float* lg;
   uint16_t* rec;  // split path: chunk records [floor(T/64) + nseq][Hv] of 17,408 bytes
-  uint16_t* y;    // split path with the gated epilogue and no y from the caller: [T, Hv, Dv]
+  uint16_t* y;    // epilogue in a kernel of its own and no y from the caller: [T, Hv, Dv]
 };
+
+bool gate_apart(int R, int Hk, int nseq, int waves);
 
 size_t carve(void* base, int R, int Hk, int T, int nseq, int waves, bool y_scratch, Workspace* w) {
   const int Hv = Hk * R;
@@ -65,10 +67,9 @@ size_t carve(void* base, int R, int Hk, int T, int nseq, int waves, bool y_scrat
   ws.lg = static_cast<float*>(take((size_t)T * Hv * 4));
   ws.rec = nullptr;
   ws.y = nullptr;
-  if (waves < 8) {
-    ws.rec = static_cast<uint16_t*>(take((size_t)(T / 64 + nseq) * Hv * kRecStride));
-    if (y_scratch) ws.y = static_cast<uint16_t*>(take((size_t)T * Hv * kDv * 2));
-  }
+  if (waves < 8) ws.rec = static_cast<uint16_t*>(take((size_t)(T / 64 + nseq) * Hv * kRecStride));
+  if (y_scratch && gate_apart(R, Hk, nseq, waves))
+    ws.y = static_cast<uint16_t*>(take((size_t)T * Hv * kDv * 2));
   if (w) *w = ws;
   return off;
 }
@@ -1292,14 +1293,15 @@ __global__ __launch_bounds__(512) void prefill_form_kernel(
     *reinterpret_cast<u32x4*>(dst + 8 * u) = *static_cast<const u32x4*>(__builtin_assume_aligned(rec_slot(sm, u), 16));
 }
 
-// Split path, RMSNormGated epilogue (qwen3_5.rs:660-665) over y written by the
-// chunk kernel: out[t, hv, :] = silu(z) * bf16(w * bf16(y * rn)). 16 lanes per
+// RMSNormGated epilogue (qwen3_5.rs:660-665) over y written by the ungated chunk
+// kernel, split or fused (gate_apart): out[t, hv, :] = silu(z) * bf16(w * bf16(y * rn)). 16 lanes per
 // (token, value head), lane j rows 8j..8j+7; the sum of y^2 runs in the order
 // of the chunk kernel's own epilogue (per 4 rows, then per 16, then over the
 // 8 groups of 16 pairwise), so that both paths give the same bits.
 __global__ __launch_bounds__(256) void prefill_norm_gate_kernel(
     const uint16_t* __restrict__ y, const uint16_t* __restrict__ zrow, int64_t xs,
-    const uint16_t* __restrict__ norm_w, float norm_eps, uint16_t* __restrict__ out, int T, int Hv) {
+    const uint16_t* __restrict__ norm_w, float norm_eps, uint16_t* __restrict__ out, int T, int Hv,
+    const int32_t* __restrict__ cu, int nseq, const int32_t* __restrict__ slot_ids, int num_slots) {
   const int item = blockIdx.x * 16 + (threadIdx.x >> 4), j = threadIdx.x & 15;
   if (item >= T * Hv) return;  // a whole 16-lane group
   const int t = item / Hv, hv = item % Hv;
@@ -1307,12 +1309,28 @@ __global__ __launch_bounds__(256) void prefill_norm_gate_kernel(
   const u32x4 yv = *reinterpret_cast<const u32x4*>(y + row);
   const u32x4 zv = *reinterpret_cast<const u32x4*>(zrow + (size_t)t * xs + (size_t)hv * kDv + 8 * j);
   const u32x4 nw = *reinterpret_cast<const u32x4*>(norm_w + 8 * j);
+  // tokens of no sequence, or of one with a bad slot, were skipped by the chunk
+  // kernel: their rows of out stay as they are. Looked up while y and z come; a
+  // wave's four items are heads of one token when Hv is a multiple of 4, and the
+  // lookup then runs on the scalar unit (on the vector memory path it cost the
+  // kernel a fifth of its rate).
+  __builtin_amdgcn_sched_barrier(0);
+  auto in_sequence = [&](int tok) {
+    const int s = seq_of(cu, nseq, tok);
+    return tok >= cu[s] && tok < cu[s + 1] && (unsigned)slot_ids[s] < (unsigned)num_slots;
+  };
+  bool live;
+  if ((Hv & 3) == 0)
+    live = in_sequence(__builtin_amdgcn_readfirstlane(t));
+  else
+    live = in_sequence(t);
   // lane 2k: rows 16k..16k+7 (the chunk kernel's lanes q = 0, 1 of wave k),
   // lane 2k + 1: rows 16k+8..16k+15 (q = 2, 3)
   float p = sumsq4(bf_lo(yv[0]), bf_hi(yv[0]), bf_lo(yv[1]), bf_hi(yv[1])) +
             sumsq4(bf_lo(yv[2]), bf_hi(yv[2]), bf_lo(yv[3]), bf_hi(yv[3]));
   p = sum16(p);  // xor 1, 2, 4, 8 partner order on DPP
-  *reinterpret_cast<u32x4*>(out + row) = norm_gate8(yv, zv, nw, rms_scale(p, norm_eps));
+  const u32x4 o = norm_gate8(yv, zv, nw, rms_scale(p, norm_eps));
+  if (live) *reinterpret_cast<u32x4*>(out + row) = o;
 }
 
 // Waves per work-group of the chunk kernel for a call: 8 runs the fused
@@ -1337,6 +1355,23 @@ static int forced_chunk_waves() {
   }
   return 0;
 }
+
+// Whether a gated call runs the RMSNormGated epilogue as a kernel of its own
+// over y (prefill_norm_gate_kernel): always on the split path, and on the fused
+// one while the chunk kernel's groups are fewer than the CUs. There the chunk
+// kernel is bound by the chain of its longest prompt, to which the epilogue in
+// the kernel adds about 2.6 us per chunk; a pass over y, z and out costs 9.6 ns
+// per chunk and sequence-head. Per gated call, epilogue in the chunk kernel
+// against apart, us: 16/32 heads six prompts of 1,000 tokens 179 / 176, four of
+// 512 92 / 86 (as split), eight of 2,048 (256 groups, in the kernel) 387 / 400;
+// 4/16 heads eight of 1 to 3,000 tokens 365 / 255.
+constexpr int kGateApartGroups = 256;
+namespace {
+bool gate_apart(int R, int Hk, int nseq, int waves) {
+  if (waves < 8) return true;
+  return forced_chunk_waves() == 0 && (int64_t)nseq * Hk * R < kGateApartGroups;
+}
+}  // namespace
 
 int prefill_chunk_waves(int R, int Hk, int nseq, int total_tokens) {
   if (const int f = forced_chunk_waves()) return total_tokens > 0 ? f : 8;
@@ -1374,7 +1409,7 @@ size_t prefill_workspace_bytes(int R, int Hk, int total_tokens, int nseq, int wa
 size_t prefill_workspace_reserve_bytes(int R, int Hk, int max_tokens) {
   // the largest call the split path takes: every sequence count it picks,
   // the gated epilogue's y scratch included
-  size_t most = prefill_workspace_bytes(R, Hk, max_tokens, 1, 8, false);
+  size_t most = prefill_workspace_bytes(R, Hk, max_tokens, 1, 8, true);
   // a forced split takes any call: up to one sequence per token
   const int f = forced_chunk_waves();
   if (f == 2 || f == 4)
@@ -1417,14 +1452,14 @@ hipError_t noalloc_scratch(void** out) {
   return hipSuccess;
 }
 
-// Split path with out: the RMSNormGated epilogue over y.
-static hipError_t launch_split_norm_gate(const PrefillArgs& a, const uint16_t* yb) {
+// The RMSNormGated epilogue over y as a kernel of its own.
+static hipError_t launch_norm_gate(const PrefillArgs& a, const uint16_t* yb) {
   const int Hv = a.Hk * a.R;
   const int D = 2 * a.Hk * kDk + Hv * kDv;
   const long items = (long)a.total_tokens * Hv;
   hipLaunchKernelGGL(prefill_norm_gate_kernel, dim3((unsigned)((items + 15) / 16)), dim3(256), 0,
                      a.stream, yb, a.mixed + D, a.xstride, a.norm_w, a.norm_eps, a.out,
-                     a.total_tokens, Hv);
+                     a.total_tokens, Hv, a.cu_seqlens, a.nseq, a.slot_ids, a.num_slots);
   return hipGetLastError();
 }
 
@@ -1443,7 +1478,7 @@ static hipError_t launch_split(const PrefillArgs& a, const Workspace& ws) {
                      a.xstride, nullptr, 0.0f, nullptr, a.status);
   e = hipGetLastError();
   if (e != hipSuccess || !a.out) return e;
-  return launch_split_norm_gate(a, yb);
+  return launch_norm_gate(a, yb);
 }
 
 // The split path in `segs` segments of whole 64-token tiles, each twice the
@@ -1522,7 +1557,7 @@ static hipError_t launch_split_pipelined(const PrefillArgs& a, const Workspace& 
   if (j == hipSuccess) j = hipStreamWaitEvent(a.stream, ev[1 + segs], 0);
   if (e == hipSuccess) e = j;
   if (e != hipSuccess || !a.out) return e;
-  return launch_split_norm_gate(a, yb);
+  return launch_norm_gate(a, yb);
 }
 
 template <int R>
@@ -1553,7 +1588,9 @@ static hipError_t launch_prefill_r(const PrefillArgs& a) {
   if (a.waves == 2) return launch_split<R, 2>(a, ws);
   if (a.waves == 4) return launch_split<R, 4>(a, ws);
   const int units = Hv * a.nseq;
-  if (a.out)
+  const bool apart = a.out && a.total_tokens > 0 && gate_apart(R, a.Hk, a.nseq, a.waves);
+  uint16_t* yb = apart && !a.y ? ws.y : a.y;
+  if (a.out && !apart)
     hipLaunchKernelGGL((prefill_chunk_kernel<R, true, 8>), dim3(units), dim3(512), 0, a.stream,
                        a.state, a.slot_ids, a.cu_seqlens, a.num_slots, a.Hk, a.total_tokens, 0,
                        a.total_tokens, ws.qn, ws.kn, ws.vc, ws.lg, ws.beta, nullptr, a.y,
@@ -1561,9 +1598,10 @@ static hipError_t launch_prefill_r(const PrefillArgs& a) {
   else
     hipLaunchKernelGGL((prefill_chunk_kernel<R, false, 8>), dim3(units), dim3(512), 0, a.stream,
                        a.state, a.slot_ids, a.cu_seqlens, a.num_slots, a.Hk, a.total_tokens, 0,
-                       a.total_tokens, ws.qn, ws.kn, ws.vc, ws.lg, ws.beta, nullptr, a.y, nullptr,
+                       a.total_tokens, ws.qn, ws.kn, ws.vc, ws.lg, ws.beta, nullptr, yb, nullptr,
                        a.xstride, nullptr, 0.0f, nullptr, a.status);
-  return hipGetLastError();
+  if ((e = hipGetLastError()) != hipSuccess || !apart) return e;
+  return launch_norm_gate(a, yb);
 }
 
 hipError_t launch_prefill(const PrefillArgs& a) {

@@ -436,6 +436,35 @@ def test_prefill_schedule_rule_edges_match_fused(gpu, prefill_waves, Hk, Hv, len
         assert np.array_equal(a, b), f"output {i} differs from the fused schedule"
 
 
+@pytest.mark.parametrize("Hk,Hv,lens", [(16, 32, [70, 200, 40]), (16, 32, [300, 600, 129])])
+def test_prefill_gated_bad_slot_leaves_its_rows(gpu, Hk, Hv, lens):
+    """A sequence with a slot id out of range is skipped whole where the
+    epilogue is a kernel of its own (fused and split schedule): its rows of
+    out keep what they held, the others' equal a call without it."""
+    import gdn_amd
+    import torch
+    say("gdn_prefill_varlen_gated bad slot", f"lens={lens}")
+    rng = np.random.default_rng(660)
+    T, D = sum(lens), conv_dim(Hk, Hv)
+    p = gen_layer_params(rng, Hk, Hv)
+    mixed, ab = gen_tokens(rng, T, Hk, Hv)
+    qkvz = np.concatenate([mixed, gen_tokens(rng, T, Hk, Hv)[0][:, :Hv * DV]], axis=1)
+    cu = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    norm_w = dev(O.f32_to_bf16(np.ones(DV, np.float32)))
+    args = (dev(qkvz), dev(ab), dev(p["A_log"]), dev(p["dt_bias"]), dev(p["conv_w"]), norm_w, 1e-6)
+    res = []
+    for slots in ([7, 0, 1], [2, 0, 1]):
+        pool = gdn_amd.Pool(1, 3, Hk, Hv)
+        out = torch.full((T, Hv, DV), -1, dtype=torch.int16, device=gpu)
+        pool.prefill_gated(0, _ids(slots), dev(cu), T, *args, out)
+        torch.cuda.synchronize()
+        res.append(host(out))
+        assert pool.check() == (1 if 7 in slots else 0)
+        pool.close()
+    assert np.all(res[0][:cu[1]] == 0xFFFF)
+    assert np.array_equal(res[0][cu[1]:], res[1][cu[1]:])
+
+
 def test_prefill_one_long_prompt_pipelined_matches_one_pass(gpu, prefill_segments):
     """One 16,384-token prompt takes the split path in 4 segments by default;
     its y, state and conv window equal the one-pass call's bit for bit, and a
