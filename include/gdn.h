@@ -577,10 +577,9 @@ gdn_status gdn_exec_logits(const gdn_exec* exec, const uint16_t** logits, int32_
  * first rotary_dim dimensions at the token's position (base rope_theta), K/V
  * appended to the cache, causal attention over the sequence's cached keys
  * (scale 1/sqrt(256)), out = attn * sigmoid(gate) per head. Head dim 256;
- * num_q_heads / num_kv_heads = 4 or 8. Results are deterministic for a given
- * step; the same tokens in a step with other sequences may differ by one bf16
- * ulp (the step's key blocks are split evenly over the workers, so a token's
- * partial sums depend on the whole step).
+ * num_q_heads / num_kv_heads = 4 or 8. Results are deterministic, and a token's
+ * are the same bits whatever else is in its step and however its prompt was
+ * cut into steps (keys are cut into partials at fixed positions).
  * ------------------------------------------------------------------------ */
 typedef struct gdn_kv_desc {
   int32_t num_layers;          /* attention layers                               */
@@ -593,7 +592,7 @@ typedef struct gdn_kv_desc {
   int32_t max_step_tokens;     /* most tokens one step appends (all sequences)   */
   int32_t device;
   int32_t max_workers;         /* waves a step's attention is split over; 0 =
-                                  1024 when each key is read about once (decode
+                                  1536 when each key is read about once (decode
                                   steps), 2048 when a step re-reads its keys
                                   (prompts); fewer when sharing the GPU        */
 } gdn_kv_desc;
