@@ -696,7 +696,8 @@ struct gdn_qlinear {
   uint16_t* sp = nullptr;    // packed scales  [Npad/16][K/128][16][2] bf16
   uint16_t* bias = nullptr;  // [Npad, G] bf16
   uint16_t* nsc = nullptr;   // [Npad, G] bf16, -128 * scales
-  float* part = nullptr;     // K-slice partials of decode-sized calls [slices][64][Npad] f32
+  int64_t part_tiles = 0;    // 64 x 128 f32 tiles of part (qlinear_part_tiles)
+  float* part = nullptr;     // partials of K-sliced calls
   uint16_t* xsum = nullptr;  // split group sums of a call's rows [kQLinearSumRows/64][3][64][G] bf16
 };
 
@@ -743,11 +744,8 @@ gdn_status gdn_qlinear_create(int32_t K, int32_t nparts, const int32_t* part_row
   q->G = K / 64;
   q->device = device;
   const size_t wbytes = (size_t)q->Npad * K / 2, gbytes = (size_t)q->Npad * q->G * 2;
-  const int slices = gdn::qlinear_decode_slices(K, q->Npad);
-  // partials of K slices: of decode-sized calls, and of tiles (K of at least two slices)
-  size_t pbytes = slices > 1 ? (size_t)slices * 64 * q->Npad * sizeof(float) : 0;
-  const size_t tbytes = (size_t)gdn::kQLinearPartTiles * 64 * 128 * sizeof(float);
-  if (K >= 1024 && 2 * (q->Npad / 128) * 2 <= gdn::kQLinearPartTiles && pbytes < tbytes) pbytes = tbytes;
+  q->part_tiles = gdn::qlinear_part_tiles(K, q->Npad);
+  const size_t pbytes = (size_t)q->part_tiles * 64 * 128 * sizeof(float);
   const size_t xbytes = (size_t)gdn::kQLinearSumRows * 3 * q->G * 2;
   // one allocation: weights, scales, biases, -128 scales (cleared: rows past N),
   // then the workspaces; every size is a multiple of 256 (Npad of 128, G of 8)
@@ -888,6 +886,7 @@ gdn_status qlinear_forward(const gdn_qlinear* q, const uint16_t* x, int64_t x_st
   a.y = y;
   a.ys = y_stride;
   a.part = q->part;
+  a.part_tiles = q->part_tiles;
   a.defer = defer;
   a.xsplit = M <= 64 ? xsplit : nullptr;
   a.xsum = q->xsum;

@@ -247,25 +247,93 @@ struct QLinearArgs {
   const uint16_t* nsc;
   uint16_t* y;        // [M, ys] bf16
   int64_t ys;
-  float* part;        // K-slice partials [slices][64][Npad] f32 (decode shapes), or null
+  float* part;        // workspace of part_tiles tiles of K-slice partials: decode sizes
+                      // [slices][64][Npad] f32, tiles [slices][tile][64 x 128]
+  int64_t part_tiles;
   QPartial* defer;    // non-null: a K-sliced call skips its slice sum and describes the
                       // partials here instead of writing y (nslice = 0 when y was written)
   const uint16_t* xsplit;  // or null: x's 64-column group sums as three bf16 parts
                            // [3][64][K/64] (launch_add_norm's), used by decode shapes
-  uint16_t* xsum;     // workspace of kQLinearSumRows rows' split sums (prefill shapes)
+  uint16_t* xsum;     // workspace of kQLinearSumRows rows' split sums
   hipStream_t stream;
 };
 // Rows whose split group sums a layer's workspace holds (a multiple of 64):
 // larger calls go in pieces of this many rows.
 constexpr int kQLinearSumRows = 16384;
 // 64 x 128 f32 tiles (32 KiB each) of a layer's partial-sum workspace: a
-// K-sliced call of M > 64 rows is at most this many work-groups.
+// K-sliced call on tiles is at most this many work-groups.
 constexpr int kQLinearPartTiles = 512;
+// Calls of at least kQLinearSumTiles tiles (three rounds of the 768 work-groups
+// that fit 256 CUs) on layers of at least kQLinearSumColumns columns form the
+// group sums once up front (qlinear_xsum_kernel) instead of in every column
+// tile: 880 us against 928 at 16384 x 2048 -> 12,352 and 199 against 215 at M =
+// 3688. Fewer tiles do not pay the extra launch (M = 300: 27.0 us against 25.3),
+// nor does a narrow layer, whose 16 column tiles share a row's sums (K = 4096 ->
+// 2048: 319 us against 309 at M = 16,384).
+constexpr int kQLinearSumTiles = 2304;
+constexpr int kQLinearSumColumns = 4096;
+constexpr int kQLinearWideN = 131072;  // decode-sized calls at least this wide use 64 x 128 tiles
+
+// K slices of a decode-sized call: one work-group per 64 columns; layers with
+// fewer than 128 such groups (out_proj: 2048 columns), and every K above 2048,
+// split K into slices of 1024 (K a multiple of 1024) or 512; very wide layers
+// take the tiled kernel.
+inline int qlinear_decode_slices(int K, int Npad) {
+  if (K <= 512 || (K <= 2048 && Npad / 64 >= 128) || Npad >= kQLinearWideN) return 1;
+  return K % 1024 == 0 ? K / 1024 : K / 512;
+}
+
+// K slices of a tile-kernel call of `tiles` 64 x 128 tiles. A work-group runs its
+// stages one after the other at about 1 us each while the chip is not full, so
+// a call with few tiles is cut along K: into the most slices that keep four
+// stages (512 k, whole sets of 8 groups) each and at most kQLinearPartTiles
+// work-groups. The slice sum is a launch of its own (3-4 us), which two slices
+// of 16 stages (K = 2048) do not pay back. Measured, unsliced against sliced:
+// K = 4096, N = 2048: M = 65 32.5 / 12.6 us (8 slices), 300 33.1 / 18.6 (4),
+// 1000 33.5 / 29.2 (2); K = 2048, N = 12,352, M = 100: 18.4 / 19.5 (2, not taken).
+inline int qlinear_tile_slices(int K, int64_t tiles) {
+  const int q = K / 512;
+  for (int s = q < 8 ? q : 8; s > (K <= 2048 ? 2 : 1); --s)
+    if (q % s == 0 && tiles * s <= kQLinearPartTiles) return s;
+  return 1;
+}
+
+// How a call of M > 0 rows runs on a layer whose partial-sum workspace holds
+// part_tiles tiles: launch_qlinear follows it, and the workspaces are sized by
+// it (qlinear_part_tiles), so that no call is cut into partials that have no room.
+struct QLinearPlan {
+  enum Kind { kWide, kDecode, kTile } kind;
+  int slices;     // K slices; above one, the f32 partials take slices * tiles tiles
+  int64_t tiles;  // 64 x 128 tiles of one slice
+  bool sums;      // group sums formed up front, unless the caller brings them (kWide)
+};
+inline QLinearPlan qlinear_plan(int K, int Npad, int M, int64_t part_tiles) {
+  const int64_t tiles = (int64_t)((M + 63) / 64) * (Npad / 128);
+  if (M <= 64 && Npad >= kQLinearWideN) return {QLinearPlan::kWide, 1, tiles, K <= 2048 && M > 32};
+  if (M <= 64) {
+    int ns = qlinear_decode_slices(K, Npad);
+    if (ns * tiles > part_tiles) ns = 1;
+    const int ksl = K / ns;  // K of a slice: the decode kernel has these three
+    if (ksl == 512 || ksl == 1024 || ksl == 2048) return {QLinearPlan::kDecode, ns, tiles, false};
+  }
+  int ns = qlinear_tile_slices(K, tiles);
+  if (ns * tiles > part_tiles) ns = 1;
+  const bool sums = ns == 1 && tiles >= kQLinearSumTiles && Npad >= kQLinearSumColumns;
+  return {QLinearPlan::kTile, ns, tiles, sums};
+}
+// The partial tiles of the layer's largest K-sliced call: over the calls of one
+// row tile and of every number of row tiles that is still cut.
+inline int64_t qlinear_part_tiles(int K, int Npad) {
+  int64_t most = 0;
+  for (int M = 64; M == 64 || 2 * (int64_t)(M / 64) * (Npad / 128) <= kQLinearPartTiles; M += 64) {
+    const QLinearPlan p = qlinear_plan(K, Npad, M, INT64_MAX);
+    if (p.slices > 1 && p.slices * p.tiles > most) most = p.slices * p.tiles;
+  }
+  return most;
+}
 
 hipError_t launch_qlinear_pack(const QLinearPackArgs& a);
 hipError_t launch_qlinear(const QLinearArgs& a);
-// K slices the decode path uses for a layer (1 = no partials workspace needed).
-int qlinear_decode_slices(int K, int Npad);
 
 hipError_t launch_decode(const DecodeArgs& a);
 hipError_t launch_recurrent(const RecurrentArgs& a);

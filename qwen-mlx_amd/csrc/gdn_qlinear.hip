@@ -31,16 +31,6 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kStageK = 128;    // k per pipeline stage: two groups
-// Calls of at least kSumTiles tiles (three rounds of the 768 work-groups that
-// fit the chip) on layers of at least kSumColumns columns form the group sums
-// once up front (qlinear_xsum_kernel) instead of in every column tile: 880 us
-// against 928 at 16384 x 2048 -> 12,352 and 199 against 215 at M = 3688. Fewer
-// tiles do not pay the extra launch (M = 300: 27.0 us against 25.3), nor does a
-// narrow layer, whose 16 column tiles share a row's sums (K = 4096 -> 2048:
-// 319 us against 309 at M = 16,384).
-constexpr int kSumTiles = 2304;
-constexpr int kSumColumns = 4096;
-constexpr int kWideDecodeN = 131072;  // decode-sized calls at least this wide use 64 x 128 tiles
 
 __device__ __forceinline__ f32x4 mfma(u32x4 a, u32x4 b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
@@ -858,35 +848,12 @@ hipError_t launch_qlinear_pack(const QLinearPackArgs& a) {
   return hipGetLastError();
 }
 
-int qlinear_decode_slices(int K, int Npad) {
-  // one work-group per 64 columns; layers with fewer than 128 such groups
-  // (out_proj: 2048 columns), and every K above 2048, split K into slices of
-  // 1024 (K a multiple of 1024) or 512; very wide layers take the tiled kernel
-  if (K <= 512 || (K <= 2048 && Npad / 64 >= 128) || Npad >= kWideDecodeN) return 1;
-  return K % 1024 == 0 ? K / 1024 : K / 512;
-}
-
-// K slices of a tile-kernel call of `tiles` 64 x 128 tiles. A work-group runs its
-// stages one after the other at about 1 us each while the chip is not full, so
-// a call with few tiles is cut along K: into the most slices that keep four
-// stages (512 k, whole sets of 8 groups) each and at most kQLinearPartTiles
-// work-groups. The slice sum is a launch of its own (3-4 us), which two slices
-// of 16 stages (K = 2048) do not pay back. Measured, unsliced against sliced:
-// K = 4096, N = 2048: M = 65 32.5 / 12.6 us (8 slices), 300 33.1 / 18.6 (4),
-// 1000 33.5 / 29.2 (2); K = 2048, N = 12,352, M = 100: 18.4 / 19.5 (2, not taken).
-int qlinear_tile_slices(int K, int64_t tiles) {
-  const int q = K / 512;
-  for (int s = q < 8 ? q : 8; s > (K <= 2048 ? 2 : 1); --s)
-    if (q % s == 0 && tiles * s <= kQLinearPartTiles) return s;
-  return 1;
-}
-
-// Tile choice: up to 64 rows (batched decode) qlinear_decode_kernel, whole K
-// (K = 512, 1024, 2048) or K slices (narrow layers, and every K above 2048 --
-// those always get a workspace); otherwise (prefill, and lm_head's decode
-// sizes) qlinear_tile_kernel's 64 x 128 tiles, cut along K where they are few
-// (qlinear_tile_slices), with the group sums formed once up front where they
-// are many (kSumTiles, kSumColumns).
+// Tile choice (qlinear_plan): up to 64 rows (batched decode) qlinear_decode_kernel,
+// whole K (K = 512, 1024, 2048) or K slices (narrow layers, and every K above
+// 2048); otherwise (prefill, lm_head's decode sizes, and K = 1536 at 8,192 columns
+// and more) qlinear_tile_kernel's 64 x 128 tiles, cut along K where they are few
+// (qlinear_tile_slices), with the group sums formed once up front where they are
+// many (kQLinearSumTiles, kQLinearSumColumns).
 //
 // Batches of up to 16 and 32 rows run the same kernels on that many rows: the
 // products, the x copies and the partial tiles shrink with the rows. In graph
@@ -917,7 +884,8 @@ int qlinear_tile_slices(int K, int64_t tiles) {
 // waves per SIMD (108-111 us) and eight-wave groups (104-105 us) were slower.
 hipError_t launch_qlinear(const QLinearArgs& a) {
   if (a.defer) *a.defer = QPartial{};
-  if (a.M <= 64 && a.Npad >= kWideDecodeN) {
+  const QLinearPlan plan = qlinear_plan(a.K, a.Npad, a.M, a.part_tiles);
+  if (plan.kind == QLinearPlan::kWide) {
     const bool xs = a.xsplit != nullptr;
     if (a.K > 2048) return xs ? launch_tile<4, 16, 1>(a) : launch_tile<4, 16, 0>(a);
     if (a.M <= 16) return xs ? launch_tile<1, 8, 1>(a) : launch_tile<1, 8, 0>(a);
@@ -926,50 +894,45 @@ hipError_t launch_qlinear(const QLinearArgs& a) {
     // column tile: 92.0 us against 93.6 at 64 x 2048 -> 248,320. Smaller ones
     // lose the launch again (16 rows 62.5 / 59.5, 32 rows 70.2 / 66.7).
     QLinearArgs c = a;
-    if (!xs) {
+    if (plan.sums && !xs) {
       hipError_t e = launch_xsum(a, a.x, a.M);
       if (e != hipSuccess) return e;
       c.xsplit = a.xsum;
     }
     return launch_tile<4, 8, 1>(c);
   }
-  if (a.M <= 64) {
-    const int ns = a.part ? qlinear_decode_slices(a.K, a.Npad) : 1;
-    const int ksl = a.K / ns;  // K of a slice
-    if (ksl == 512 || ksl == 1024 || ksl == 2048) {
-      const u32x4* wp = reinterpret_cast<const u32x4*>(a.wp);
-      const bool xs = a.xsplit != nullptr && ns == 1 && ksl == 2048;
-      auto pick = [&](auto mu) {
-        constexpr int MU = decltype(mu)::value;
-        return xs            ? qlinear_decode_kernel<8, 2, MU, true>
-               : ksl == 2048 ? qlinear_decode_kernel<8, 2, MU, false>
-               : ksl == 1024 ? qlinear_decode_kernel<8, 1, MU, false>
-                             : qlinear_decode_kernel<4, 1, MU, false>;
-      };
-      auto kern = a.M <= 16   ? pick(std::integral_constant<int, 1>{})
-                  : a.M <= 32 ? pick(std::integral_constant<int, 2>{})
-                              : pick(std::integral_constant<int, 4>{});
-      const int threads = ksl == 512 ? 256 : 512;
-      hipLaunchKernelGGL(kern, dim3(a.Npad / 64, ns), dim3(threads), 0, a.stream, a.x, a.xs, a.M,
-                         a.K, wp, a.sp, a.bias, a.nsc, a.N, a.y, a.ys, ns > 1 ? a.part : nullptr,
-                         a.Npad, xs ? a.xsplit : nullptr);
-      hipError_t e = hipGetLastError();
-      if (e != hipSuccess || ns == 1) return e;
-      if (a.defer) {  // the consumer adds the slices
-        *a.defer = QPartial{a.part, ns, a.Npad};
-        return hipSuccess;
-      }
-      const int64_t n4 = (int64_t)a.M * (a.Npad / 4);
-      hipLaunchKernelGGL(qlinear_sum_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0,
-                         a.stream, a.part, ns, a.M, a.N, a.Npad, a.y, a.ys);
-      return hipGetLastError();
+  if (plan.kind == QLinearPlan::kDecode) {
+    const int ns = plan.slices, ksl = a.K / ns;  // K of a slice
+    const u32x4* wp = reinterpret_cast<const u32x4*>(a.wp);
+    const bool xs = a.xsplit != nullptr && ns == 1 && ksl == 2048;
+    auto pick = [&](auto mu) {
+      constexpr int MU = decltype(mu)::value;
+      return xs            ? qlinear_decode_kernel<8, 2, MU, true>
+             : ksl == 2048 ? qlinear_decode_kernel<8, 2, MU, false>
+             : ksl == 1024 ? qlinear_decode_kernel<8, 1, MU, false>
+                           : qlinear_decode_kernel<4, 1, MU, false>;
+    };
+    auto kern = a.M <= 16   ? pick(std::integral_constant<int, 1>{})
+                : a.M <= 32 ? pick(std::integral_constant<int, 2>{})
+                            : pick(std::integral_constant<int, 4>{});
+    const int threads = ksl == 512 ? 256 : 512;
+    hipLaunchKernelGGL(kern, dim3(a.Npad / 64, ns), dim3(threads), 0, a.stream, a.x, a.xs, a.M,
+                       a.K, wp, a.sp, a.bias, a.nsc, a.N, a.y, a.ys, ns > 1 ? a.part : nullptr,
+                       a.Npad, xs ? a.xsplit : nullptr);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || ns == 1) return e;
+    if (a.defer) {  // the consumer adds the slices
+      *a.defer = QPartial{a.part, ns, a.Npad};
+      return hipSuccess;
     }
+    const int64_t n4 = (int64_t)a.M * (a.Npad / 4);
+    hipLaunchKernelGGL(qlinear_sum_kernel, dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0,
+                       a.stream, a.part, ns, a.M, a.N, a.Npad, a.y, a.ys);
+    return hipGetLastError();
   }
-  const int64_t tiles = (int64_t)((a.M + 63) / 64) * (a.Npad / 128);
-  const int slices = qlinear_tile_slices(a.K, tiles);
-  if (slices > 1 || tiles < kSumTiles || a.Npad < kSumColumns) {
-    if (a.K / slices <= 2048) return launch_tile<4, 8, 0>(a, slices);
-    return launch_tile<4, 16, 0>(a, slices);
+  if (!plan.sums) {
+    if (a.K / plan.slices <= 2048) return launch_tile<4, 8, 0>(a, plan.slices);
+    return launch_tile<4, 16, 0>(a, plan.slices);
   }
   QLinearArgs c = a;
   for (int m = 0; m < a.M; m += kQLinearSumRows) {

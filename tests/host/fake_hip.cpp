@@ -143,15 +143,14 @@ hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
 namespace gdn {
 
 hipError_t launch_qlinear_pack(const QLinearPackArgs&) { return hipSuccess; }
-int qlinear_decode_slices(int K, int Npad) {
-  if (K <= 512 || (K <= 2048 && Npad / 64 >= 128) || Npad >= 131072) return 1;
-  return K / 512;
-}
+// A K-sliced call clears its partials to their last element, as the kernels
+// write them, so that a workspace which is missing or too small shows.
 hipError_t launch_qlinear(const QLinearArgs& a) {
   if (a.defer) *a.defer = QPartial{};
-  if (a.M <= 64 && a.Npad < 131072 && a.part) {
-    const int ns = qlinear_decode_slices(a.K, a.Npad);
-    if (ns > 1 && a.defer) *a.defer = QPartial{a.part, ns, a.Npad};
+  const QLinearPlan p = qlinear_plan(a.K, a.Npad, a.M, a.part_tiles);
+  if (p.slices > 1) {
+    std::memset(a.part, 0, (size_t)p.slices * p.tiles * 64 * 128 * sizeof(float));
+    if (p.kind == QLinearPlan::kDecode && a.defer) *a.defer = QPartial{a.part, p.slices, a.Npad};
   }
   return hipSuccess;
 }

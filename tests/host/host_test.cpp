@@ -1,14 +1,16 @@
-// Host-code test of libgdn under AddressSanitizer / UBSan: the pool's slot
-// allocator, argument checks, the debug slot-list check, the KV cache's page
+// Host-code test of libgdn under AddressSanitizer / UBSan: the projections'
+// dispatch rule against their workspaces, the pool's slot allocator, argument checks, the debug slot-list check, the KV cache's page
 // planner and accounting, and the executor's admission, batching, error and
 // rollback paths, run against the runtime stand-in in fake_hip.cpp (no GPU;
 // kernels compute nothing). Exits 0 and prints "ALL OK" when every check holds.
+#include <algorithm>
 #include <cstdint>
 #include <cstdio>
 #include <cstring>
 #include <vector>
 
 #include "gdn.h"
+#include "gdn_common.h"
 
 namespace gdn_fake {
 extern bool fail_embed;  // fake_hip.cpp: the next embedding launches fail
@@ -49,6 +51,40 @@ static gdn_qlinear* make_qlinear(std::vector<std::vector<char>>& keep, int K,
                          nullptr, &q) != GDN_OK)
     return nullptr;
   return q;
+}
+
+// Every K-sliced call has room for its partials and every layer only as many
+// as its largest call takes, over all K, widths and row counts; and a layer
+// without partials is never cut.
+static int test_qlinear_plan() {
+  std::vector<int> rows = {1, 16, 64};
+  for (int M = 65; M <= 16640; M += 64) rows.push_back(M);
+  rows.push_back(8388480);
+  for (int K = 512; K <= 4096; K += 512)
+    for (int Npad = 128; Npad <= 200064; Npad += 128) {
+      const int64_t room = gdn::qlinear_part_tiles(K, Npad);
+      int64_t most = 0;
+      bool ok = true;
+      for (int M : rows) {
+        const gdn::QLinearPlan p = gdn::qlinear_plan(K, Npad, M, room);
+        ok = ok && p.slices == gdn::qlinear_plan(K, Npad, M, INT64_MAX).slices;
+        ok = ok && gdn::qlinear_plan(K, Npad, M, 0).slices == 1 && !(p.sums && p.slices > 1);
+        if (p.slices > 1) most = std::max(most, p.slices * p.tiles);
+      }
+      if (!ok || most != room) std::fprintf(stderr, "K = %d, Npad = %d\n", K, Npad);
+      CHECK(ok && most == room);
+    }
+  // the same through the entry points: the stand-in launch writes the partials
+  std::vector<std::vector<char>> keep;
+  for (int N : {400, 8192, 16384, 16400, 21760, 21776}) {
+    gdn_qlinear* q = make_qlinear(keep, 1536, {N});
+    CHECK(q);
+    uint16_t* x = dev_alloc<uint16_t>(keep, 130 * 1536);
+    uint16_t* y = dev_alloc<uint16_t>(keep, (size_t)130 * N);
+    for (int M : {1, 64, 65, 130}) CHECK(gdn_qlinear_forward(q, x, 1536, M, y, N, nullptr) == GDN_OK);
+    CHECK(gdn_qlinear_destroy(q) == GDN_OK);
+  }
+  return 0;
 }
 
 static int test_pool() {
@@ -351,7 +387,7 @@ static int test_exec_graphs_follow_pool_buffer() {
 }
 
 int main() {
-  if (test_pool() || test_kv() || test_exec() || test_exec_graphs_follow_pool_buffer()) return 1;
+  if (test_qlinear_plan() || test_pool() || test_kv() || test_exec() || test_exec_graphs_follow_pool_buffer()) return 1;
   std::printf("ALL OK (%d checks)\n", g_checks);
   return 0;
 }

@@ -202,6 +202,9 @@ def test_qlinear_small_batches_match_full_batch(gpu, M, K, rows):
     (65, 2048, 9216),     # K = 2048: two slices would fit and are not taken
     (2241, 4096, 8208),   # up-front group sums of 64 groups, one row in the last row tile
     (16449, 512, 4112),   # more rows than one piece of the up-front sums
+    (1, 1536, 16400),     # decode sizes on tiles: 129 tiles in 3 slices
+    (64, 1536, 16400),
+    (64, 1536, 21888),    # 171 tiles: no longer cut
 ])
 def test_qlinear_tiles_and_slices_sampled(gpu, M, K, N):
     """The tile kernel's K slices and up-front group sums at the edges of
