@@ -298,11 +298,13 @@ typedef struct gdn_qlinear gdn_qlinear;
 /* Merge nparts MLX-format parts (device pointers, part i has part_rows[i]
  * output rows) into one layer with N = sum(part_rows) outputs and repack it
  * for the kernel on `device`. The layer owns its memory: about N*K/2 +
- * 3*N*K/32 bytes; 16384 * 3*K/32 bytes for a call's group sums; and for layers
- * whose calls can split K (K >= 1024 and N <= 16384, or K > 2048) f32 partial
- * sums, 16 MiB or K/512 * 64 * N of them if that is more. The sources are only read, and may be freed once this returns (it synchronises
- * `stream`). Supported: bits 4, group_size 64, K a multiple of 512 up to
- * 4096, part_rows multiples of 16. */
+ * 3*N*K/32 bytes; on layers of more than 3,968 columns 16384 * 3*K/32 bytes for
+ * a call's group sums; and on layers some calls of which split K (K above 2048
+ * below 131,072 columns, K = 2048 up to 8,192, K = 1536 up to 21,760) the f32
+ * partial sums of the largest such call, at most 16 MiB or K/512 * 64 * N of
+ * them if that is more. The sources are only read, and may be freed once this
+ * returns (it synchronises `stream`). Supported: bits 4, group_size 64, K a
+ * multiple of 512 up to 4096, part_rows multiples of 16. */
 gdn_status gdn_qlinear_create(int32_t K, int32_t nparts, const int32_t* part_rows,
                               const uint32_t* const* w, const uint16_t* const* scales,
                               const uint16_t* const* biases, int32_t group_size, int32_t bits,
@@ -316,7 +318,8 @@ gdn_status gdn_qlinear_dims(const gdn_qlinear* layer, int32_t* K, int32_t* N);
  * (columns past N untouched). x: 16-byte aligned, x_stride >= K and a
  * multiple of 8; y: 8-byte aligned, y_stride >= N and a multiple of 4;
  * M <= 8,388,480. Allocates nothing. Calls on one layer must be ordered on
- * one stream (a K-split call uses the layer's partial-sum buffer). For the
+ * one stream: any of them may use the layer's workspaces (group sums and
+ * partial sums), also on layers whose calls never split K. For the
  * merged qkv|z|b|a layer the
  * output row is [q|k|v|z|b|a], which gdn_decode_gated reads in place
  * (qkvz = y, row_stride = y_stride; ab = y + D + Hv*Dv, ab_stride = y_stride). */

@@ -698,7 +698,8 @@ struct gdn_qlinear {
   uint16_t* nsc = nullptr;   // [Npad, G] bf16, -128 * scales
   int64_t part_tiles = 0;    // 64 x 128 f32 tiles of part (qlinear_part_tiles)
   float* part = nullptr;     // partials of K-sliced calls
-  uint16_t* xsum = nullptr;  // split group sums of a call's rows [kQLinearSumRows/64][3][64][G] bf16
+  uint16_t* xsum = nullptr;  // split group sums of a call's rows [kQLinearSumRows/64][3][64][G]
+                             // bf16 on layers some call of which forms them up front
 };
 
 static void qlinear_release(gdn_qlinear* q) {
@@ -746,7 +747,8 @@ gdn_status gdn_qlinear_create(int32_t K, int32_t nparts, const int32_t* part_row
   const size_t wbytes = (size_t)q->Npad * K / 2, gbytes = (size_t)q->Npad * q->G * 2;
   q->part_tiles = gdn::qlinear_part_tiles(K, q->Npad);
   const size_t pbytes = (size_t)q->part_tiles * 64 * 128 * sizeof(float);
-  const size_t xbytes = (size_t)gdn::kQLinearSumRows * 3 * q->G * 2;
+  const size_t xbytes =
+      q->Npad >= gdn::kQLinearSumColumns ? (size_t)gdn::kQLinearSumRows * 3 * q->G * 2 : 0;
   // one allocation: weights, scales, biases, -128 scales (cleared: rows past N),
   // then the workspaces; every size is a multiple of 256 (Npad of 128, G of 8)
   const size_t cleared = wbytes + 3 * gbytes;
@@ -762,7 +764,7 @@ gdn_status gdn_qlinear_create(int32_t K, int32_t nparts, const int32_t* part_row
   q->bias = reinterpret_cast<uint16_t*>(base + wbytes + gbytes);
   q->nsc = reinterpret_cast<uint16_t*>(base + wbytes + 2 * gbytes);
   if (pbytes) q->part = reinterpret_cast<float*>(base + cleared);
-  q->xsum = reinterpret_cast<uint16_t*>(base + cleared + pbytes);
+  if (xbytes) q->xsum = reinterpret_cast<uint16_t*>(base + cleared + pbytes);
   hipStream_t s = as_stream(stream);
   hipError_t e;
   if ((e = hipMemsetAsync(q->wp, 0, cleared, s)) != hipSuccess) {

@@ -22,6 +22,7 @@ namespace gdn_fake {
 bool fail_embed = false;  // set by the test: embedding launches fail
 bool capture = false;     // set by the test: stream capture records the stand-in launches
 bool split = false;       // set by the test: prefill calls take the split path (2-wave groups)
+size_t malloc_bytes = 0;  // size of the last hipMalloc
 int graphs_live = 0, graphs_destroyed = 0, graphs_made = 0;
 std::vector<std::function<void()>>* recording = nullptr;  // the capture in progress
 }
@@ -29,6 +30,7 @@ std::vector<std::function<void()>>* recording = nullptr;  // the capture in prog
 extern "C" {
 
 hipError_t hipMalloc(void** ptr, size_t size) {
+  gdn_fake::malloc_bytes = size;
   *ptr = std::calloc(1, size ? size : 1);
   return *ptr ? hipSuccess : hipErrorOutOfMemory;
 }
@@ -143,8 +145,9 @@ hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
 namespace gdn {
 
 hipError_t launch_qlinear_pack(const QLinearPackArgs&) { return hipSuccess; }
-// A K-sliced call clears its partials to their last element, as the kernels
-// write them, so that a workspace which is missing or too small shows.
+// A K-sliced call clears its partials to their last element and a call that
+// forms its group sums up front those of its first rows, as the kernels write
+// them, so that a workspace which is missing or too small shows.
 hipError_t launch_qlinear(const QLinearArgs& a) {
   if (a.defer) *a.defer = QPartial{};
   const QLinearPlan p = qlinear_plan(a.K, a.Npad, a.M, a.part_tiles);
@@ -152,6 +155,8 @@ hipError_t launch_qlinear(const QLinearArgs& a) {
     std::memset(a.part, 0, (size_t)p.slices * p.tiles * 64 * 128 * sizeof(float));
     if (p.kind == QLinearPlan::kDecode && a.defer) *a.defer = QPartial{a.part, p.slices, a.Npad};
   }
+  if (p.sums && !a.xsplit)
+    std::memset(a.xsum, 0, (size_t)std::min((a.M + 63) / 64 * 64, kQLinearSumRows) * 3 * (a.K / 64) * 2);
   return hipSuccess;
 }
 hipError_t launch_decode(const DecodeArgs&) { return hipSuccess; }

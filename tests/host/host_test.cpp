@@ -16,6 +16,7 @@ namespace gdn_fake {
 extern bool fail_embed;  // fake_hip.cpp: the next embedding launches fail
 extern bool capture;     // fake_hip.cpp: stream capture makes (empty) graphs
 extern bool split;       // fake_hip.cpp: prefill calls take the split path
+extern size_t malloc_bytes;  // fake_hip.cpp: size of the last device allocation
 extern int graphs_live, graphs_destroyed, graphs_made;
 }
 
@@ -82,6 +83,23 @@ static int test_qlinear_plan() {
     uint16_t* x = dev_alloc<uint16_t>(keep, 130 * 1536);
     uint16_t* y = dev_alloc<uint16_t>(keep, (size_t)130 * N);
     for (int M : {1, 64, 65, 130}) CHECK(gdn_qlinear_forward(q, x, 1536, M, y, N, nullptr) == GDN_OK);
+    CHECK(gdn_qlinear_destroy(q) == GDN_OK);
+  }
+  // what a layer holds beyond its weights: K = 2048 of 12,352 columns is never
+  // cut (group sums only), K = 4096 of 2,048 never forms its sums up front
+  // (partials only), K = 512 of 400 does neither
+  struct {
+    int K, N, M;
+    size_t extra;
+  } cases[] = {{2048, 12352, 16384, 16384 * 3 * 32 * 2}, {4096, 2048, 960, 512 * 32768}, {512, 400, 65, 0}};
+  for (const auto& c : cases) {
+    gdn_qlinear* q = make_qlinear(keep, c.K, {c.N});
+    CHECK(q);
+    const size_t npad = (c.N + 127) / 128 * 128;
+    CHECK(gdn_fake::malloc_bytes == npad * c.K / 2 + 3 * npad * (c.K / 64) * 2 + c.extra);
+    uint16_t* x = dev_alloc<uint16_t>(keep, (size_t)c.M * c.K);
+    uint16_t* y = dev_alloc<uint16_t>(keep, (size_t)c.M * c.N);
+    CHECK(gdn_qlinear_forward(q, x, c.K, c.M, y, c.N, nullptr) == GDN_OK);
     CHECK(gdn_qlinear_destroy(q) == GDN_OK);
   }
   return 0;
