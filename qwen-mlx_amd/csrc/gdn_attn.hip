@@ -510,10 +510,11 @@ __global__ __launch_bounds__(512, 2) void attn_tile_kernel(
 
   auto block = [&](int kb, auto bc) {
     constexpr int b = decltype(bc)::value;
-    // this wave's copies of block kb have landed; after the barrier everyone's
-    // have, and everyone is done with the other buffer
+    // this wave's copies of block kb have landed and its reads of the other
+    // buffer have returned (lds_barrier waits for them): after the barrier
+    // everyone's have, and the other buffer may be copied over
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
-    __builtin_amdgcn_s_barrier();
+    lds_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup", "global");
     copy(min(kb + 1, nblk - 1), std::integral_constant<int, 1 - b>{});
     __builtin_amdgcn_sched_barrier(0);
