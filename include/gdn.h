@@ -594,10 +594,11 @@ typedef struct gdn_kv_desc {
   int32_t head_dim;            /* must be 256                                    */
   int32_t max_step_tokens;     /* most tokens one step appends (all sequences)   */
   int32_t device;
-  int32_t max_workers;         /* waves a step's attention is split over; 0 =
-                                  1536 when each key is read about once (decode
-                                  steps), 2048 when a step re-reads its keys
-                                  (prompts); fewer when sharing the GPU        */
+  int32_t max_workers;         /* most waves a step's attention is split over,
+                                  for sharing the GPU; 0 = no limit: 1536 when
+                                  each key is read about once (decode steps),
+                                  2048 when a step re-reads its keys (prompts),
+                                  and larger prompts in tiles over the chip     */
 } gdn_kv_desc;
 
 /* Per layer num_pages x 128 KiB of bf16 K/V (at 2 kv heads), a page table,

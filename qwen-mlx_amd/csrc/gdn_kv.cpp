@@ -287,7 +287,8 @@ gdn_status gdn_kv_step(gdn_kv* kv, int32_t n, const int32_t* slots, const int32_
         longest = std::max(longest, nb);
       }
     }
-    const bool tiled = use_tiles(work, longest);
+    // a limit on the workers holds for prompts too: they stay on chunks
+    const bool tiled = d.max_workers == 0 && use_tiles(work, longest);
     int32_t t0 = 0;
     for (int i = 0; i < n; ++i) {
       const bool tile = tiled && ntok[i] >= kTileMinTokens;

@@ -22,6 +22,7 @@ namespace gdn_fake {
 bool fail_embed = false;  // set by the test: embedding launches fail
 bool capture = false;     // set by the test: stream capture records the stand-in launches
 bool split = false;       // set by the test: prefill calls take the split path (2-wave groups)
+gdn::AttnArgs attn;       // of the last attention launch
 size_t malloc_bytes = 0;  // size of the last hipMalloc
 int graphs_live = 0, graphs_destroyed = 0, graphs_made = 0;
 std::vector<std::function<void()>>* recording = nullptr;  // the capture in progress
@@ -190,7 +191,10 @@ size_t attn_workspace_bytes(int T, int Hq, int64_t chunks) {
 }
 int attn_chunk_keys() { return 384; }
 int attn_block_keys() { return 32; }
-hipError_t launch_attn(const AttnArgs&) { return hipSuccess; }
+hipError_t launch_attn(const AttnArgs& a) {
+  gdn_fake::attn = a;
+  return hipSuccess;
+}
 hipError_t launch_kv_gather(const uint16_t*, const int32_t*, int, int64_t, uint16_t*, uint16_t*,
                             hipStream_t) {
   return hipSuccess;

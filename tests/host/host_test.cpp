@@ -16,6 +16,7 @@ namespace gdn_fake {
 extern bool fail_embed;  // fake_hip.cpp: the next embedding launches fail
 extern bool capture;     // fake_hip.cpp: stream capture makes (empty) graphs
 extern bool split;       // fake_hip.cpp: prefill calls take the split path
+extern gdn::AttnArgs attn;  // fake_hip.cpp: arguments of the last attention launch
 extern size_t malloc_bytes;  // fake_hip.cpp: size of the last device allocation
 extern int graphs_live, graphs_destroyed, graphs_made;
 }
@@ -220,6 +221,32 @@ static int test_kv() {
   return 0;
 }
 
+// A caller's max_workers bounds prompt steps as well as decode steps; without
+// one a prompt that fills the chip runs as tiles.
+static int test_kv_max_workers() {
+  std::vector<std::vector<char>> keep;
+  const int Hq = 16, Hkv = 2, T = 2048;
+  uint16_t* q = dev_alloc<uint16_t>(keep, (size_t)T * Hq * 512);
+  uint16_t* k = dev_alloc<uint16_t>(keep, (size_t)T * Hkv * 256);
+  uint16_t* w = dev_alloc<uint16_t>(keep, 256);
+  uint16_t* out = dev_alloc<uint16_t>(keep, (size_t)T * Hq * 256);
+  for (int workers : {0, 1, 64}) {
+    gdn_kv_desc d{1, 2, 80, 40, Hq, Hkv, 256, T, 0, workers};
+    gdn_kv* kv = nullptr;
+    CHECK(gdn_kv_create(&d, &kv) == GDN_OK);
+    const int32_t slot = 1;
+    for (int32_t n : {T, 1}) {
+      CHECK(gdn_kv_step(kv, 1, &slot, &n, nullptr) == GDN_OK);
+      CHECK(gdn_attn_forward(kv, 0, q, Hq * 512, k, Hkv * 256, k, Hkv * 256, w, w, 1e-6f, 1e6f, 64,
+                             out, Hq * 256, nullptr) == GDN_OK);
+      CHECK((gdn_fake::attn.NT > 0) == (workers == 0 && n > 1));
+      if (workers) CHECK(gdn_fake::attn.P >= 1 && gdn_fake::attn.P <= workers);
+    }
+    CHECK(gdn_kv_destroy(kv) == GDN_OK);
+  }
+  return 0;
+}
+
 static int test_exec() {
   std::vector<std::vector<char>> keep;
   const int hidden = 512, vocab = 1024, Hk = 16, Hv = 32, D = 2 * Hk * 128 + Hv * 128;
@@ -405,7 +432,9 @@ static int test_exec_graphs_follow_pool_buffer() {
 }
 
 int main() {
-  if (test_qlinear_plan() || test_pool() || test_kv() || test_exec() || test_exec_graphs_follow_pool_buffer()) return 1;
+  if (test_qlinear_plan() || test_pool() || test_kv() || test_kv_max_workers() || test_exec() ||
+      test_exec_graphs_follow_pool_buffer())
+    return 1;
   std::printf("ALL OK (%d checks)\n", g_checks);
   return 0;
 }
