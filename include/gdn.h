@@ -41,10 +41,15 @@
  *     ordered on one stream by the caller. gdn_prefill_varlen uses a device
  *     workspace held by the pool, so its calls on a pool must be ordered on
  *     one stream; a call that needs more workspace than the pool holds
- *     (it grows with total_tokens, and for a few long sequences also holds
- *     their chunk records) synchronizes its stream and reallocates it, later
+ *     (it grows with total_tokens; calls on the split schedule also hold their
+ *     chunk records there, and gated calls may hold their ungated rows)
+ *     synchronizes its stream and reallocates it, later
  *     calls at or below that size allocate nothing; gdn_pool_reserve sizes it
- *     for any call up to a token count. gdn_decode allocates nothing.
+ *     for any call up to a token count. Under stream capture, and when the
+ *     device has no memory left, such a call takes the schedule with the
+ *     smallest workspace instead (16,576 bytes per token at 16 key / 32 value
+ *     heads; the same bits) and grows the buffer only if that does not fit,
+ *     which a capture does not survive. gdn_decode allocates nothing.
  *   - The decode entries launch kernels only (no memset nodes, no host
  *     synchronisation), so a decode step over every layer can be captured in
  *     one HIP graph and replayed: gdn_decode, gdn_decode_gated, gdn_recurrent,
@@ -225,7 +230,8 @@ gdn_status gdn_decode_gated(gdn_pool* pool, int32_t layer, const int32_t* slot_i
  * sequence-heads), the chunks'
  * state-independent blocks formed for all chunks at once and 2 or 4
  * work-groups per (sequence, value head). The environment variable
- * GDN_PREFILL_WAVES = 8 (the first), 4 or 2 (the second) forces one.
+ * GDN_PREFILL_WAVES = 8 (the first), 4 or 2 (the second) forces one where its
+ * workspace can be had.
  * The second schedule, for one sequence of at least 8,192 tokens and at most
  * half as many work-groups as the device has CUs (one 16,384-token prompt at
  * 32 value heads: 128), runs as a pipeline of 2 to 8 token segments (each

@@ -430,6 +430,14 @@ static gdn_status ensure_workspace(gdn_pool* pool, size_t need, void* stream, co
   return ensure_buffer(pool->workspace, pool->workspace_bytes, need, stream, what);
 }
 
+// Whether a stream is being captured (or cannot be asked).
+static bool capturing(hipStream_t stream) {
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(stream, &cs) == hipSuccess) return cs != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
 // The pool's second stream and events for a pipelined prefill (default
 // priority, not blocking on the null stream), made once on the pool's device.
 // false when they cannot be made: the call then runs in one pass.
@@ -562,31 +570,40 @@ static gdn_status prefill_common(gdn_pool* pool, int32_t layer, const int32_t* s
   DeviceGuard guard(pool->d.device);
   st = debug_check_slots(pool, slot_ids, nseq, stream, who);
   if (st) return st;
-  // The no-allocation entry takes the library's schedule when its workspace
-  // fits the fixed scratch, and otherwise the fused schedule, whose workspace
-  // is the smallest.
-  int waves = gdn::prefill_chunk_waves(pool->R, pool->d.num_k_heads, nseq, total_tokens);
-  size_t need = gdn::prefill_workspace_bytes(pool->R, pool->d.num_k_heads, total_tokens, nseq,
-                                             waves, out && !y);
-  if (noalloc && waves != 8 && need > gdn::noalloc_scratch_bytes()) {
+  // The library's schedule where its workspace fits or can be had; otherwise
+  // the fused one with the gated epilogue in its chunk kernel, whose workspace
+  // is the smallest (the same bits): in the no-allocation entry, under capture
+  // (where the pool's buffer cannot grow), and when the device has no memory left.
+  const int R = pool->R, Hk = pool->d.num_k_heads;
+  int waves = gdn::prefill_chunk_waves(R, Hk, nseq, total_tokens);
+  bool apart = out && total_tokens > 0 && gdn::prefill_gate_apart(R, Hk, nseq, waves, pool->cus);
+  size_t need = gdn::prefill_workspace_bytes(R, Hk, total_tokens, nseq, waves, apart && !y);
+  const size_t least = gdn::prefill_workspace_bytes(R, Hk, total_tokens, nseq, 8, false);
+  auto smallest = [&] {
     waves = 8;
-    need = gdn::prefill_workspace_bytes(pool->R, pool->d.num_k_heads, total_tokens, nseq, waves,
-                                        out && !y);
-  }
+    apart = false;
+    need = least;
+  };
   void* ws = nullptr;
   size_t ws_bytes = 0;
   if (noalloc) {
     ws_bytes = gdn::noalloc_scratch_bytes();
+    if (need > ws_bytes) smallest();
     if (need > ws_bytes)
       return fail(GDN_ERR_INVALID,
                   "%s: %d tokens need %zu bytes of workspace; its fixed scratch holds %zu "
                   "(%zu bytes per token at these head counts)",
                   who, total_tokens, need, ws_bytes,
-                  gdn::prefill_workspace_bytes(pool->R, pool->d.num_k_heads, 1, 1, 8, false));
+                  gdn::prefill_workspace_bytes(R, Hk, 1, 1, 8, false));
     hipError_t e = gdn::noalloc_scratch(&ws);
     if (e != hipSuccess) return hip_fail(e, "hipGetSymbolAddress(scratch)");
   } else {
+    if (need > pool->workspace_bytes && capturing(as_stream(stream))) smallest();
     st = ensure_workspace(pool, need, stream, "prefill");
+    if (st == GDN_ERR_OOM && need > least) {
+      smallest();
+      st = ensure_workspace(pool, need, stream, "prefill");
+    }
     if (st) return st;
     ws = pool->workspace;
     ws_bytes = pool->workspace_bytes;
@@ -614,6 +631,7 @@ static gdn_status prefill_common(gdn_pool* pool, int32_t layer, const int32_t* s
   a.out = out;
   a.status = pool->d_status;
   a.waves = waves;
+  a.apart = apart;
   a.workspace = ws;
   a.workspace_bytes = ws_bytes;
   a.stream = as_stream(stream);
@@ -621,17 +639,10 @@ static gdn_status prefill_common(gdn_pool* pool, int32_t layer, const int32_t* s
   // stream capture and in the no-allocation entry (which makes no objects).
   const int groups = pool->d.num_v_heads * nseq * (waves ? 8 / waves : 1);
   const int segs = gdn::prefill_pipeline_segments(waves, nseq, total_tokens, groups, pool->cus);
-  if (!noalloc && segs > 1) {
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(a.stream, &cs) != hipSuccess) {
-      (void)hipGetLastError();
-      cs = hipStreamCaptureStatusActive;
-    }
-    if (cs == hipStreamCaptureStatusNone && ensure_pipeline(pool)) {
-      a.aux = pool->aux;
-      a.events = pool->pipe_ev;
-      a.segments = segs;
-    }
+  if (!noalloc && segs > 1 && !capturing(a.stream) && ensure_pipeline(pool)) {
+    a.aux = pool->aux;
+    a.events = pool->pipe_ev;
+    a.segments = segs;
   }
   hipError_t e = gdn::launch_prefill(a);
   if (e != hipSuccess) return hip_fail(e, who);
@@ -1001,7 +1012,8 @@ gdn_status gdn_pool_reserve(gdn_pool* pool, int32_t max_tokens, void* stream) {
                      "layer activation", &pool->act_gen);
   if (st) return st;
   return ensure_workspace(pool, gdn::prefill_workspace_reserve_bytes(pool->R, pool->d.num_k_heads,
-                                                                     max_tokens), stream, "prefill");
+                                                                     max_tokens, pool->cus),
+                          stream, "prefill");
 }
 
 gdn_status gdn_layer_decode(gdn_layer* L, const int32_t* slot_ids, int32_t B, const uint16_t* x,

@@ -201,6 +201,7 @@ struct PrefillArgs {
   uint16_t* out;          // [T, Hv, Dv] = silu(z) * rms_norm(y), or null
   uint32_t* status;
   int waves;             // prefill_chunk_waves of the call (8: fused chunk kernel)
+  bool apart;            // the gated epilogue runs as a kernel of its own over y
   void* workspace;       // device scratch sized by prefill_workspace_bytes
   size_t workspace_bytes;
   hipStream_t stream;
@@ -345,8 +346,10 @@ int prefill_chunk_waves(int R, int Hk, int nseq, int total_tokens);
 // chunk kernel has `groups` work-groups, on a device of `cus` CUs (1: one
 // pass, no second stream).
 int prefill_pipeline_segments(int waves, int nseq, int total_tokens, int groups, int cus);
+bool prefill_gate_apart(int R, int Hk, int nseq, int waves, int cus);
+// y_scratch: the epilogue runs apart and the caller brings no y.
 size_t prefill_workspace_bytes(int R, int Hk, int total_tokens, int nseq, int waves, bool y_scratch);
-size_t prefill_workspace_reserve_bytes(int R, int Hk, int max_tokens);
+size_t prefill_workspace_reserve_bytes(int R, int Hk, int max_tokens, int cus);
 // Fixed per-device workspace of gdn_prefill_varlen_noalloc (gdn_prefill.hip).
 size_t noalloc_scratch_bytes();
 hipError_t noalloc_scratch(void** out);

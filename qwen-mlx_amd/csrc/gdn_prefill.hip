@@ -48,8 +48,6 @@ struct Workspace {
   uint16_t* y;    // epilogue in a kernel of its own and no y from the caller: [T, Hv, Dv]
 };
 
-bool gate_apart(int R, int Hk, int nseq, int waves);
-
 size_t carve(void* base, int R, int Hk, int T, int nseq, int waves, bool y_scratch, Workspace* w) {
   const int Hv = Hk * R;
   size_t off = 0;
@@ -68,7 +66,7 @@ size_t carve(void* base, int R, int Hk, int T, int nseq, int waves, bool y_scrat
   ws.rec = nullptr;
   ws.y = nullptr;
   if (waves < 8) ws.rec = static_cast<uint16_t*>(take((size_t)(T / 64 + nseq) * Hv * kRecStride));
-  if (y_scratch && gate_apart(R, Hk, nseq, waves))
+  if (y_scratch)
     ws.y = static_cast<uint16_t*>(take((size_t)T * Hv * kDv * 2));
   if (w) *w = ws;
   return off;
@@ -1294,7 +1292,7 @@ __global__ __launch_bounds__(512) void prefill_form_kernel(
 }
 
 // RMSNormGated epilogue (qwen3_5.rs:660-665) over y written by the ungated chunk
-// kernel, split or fused (gate_apart): out[t, hv, :] = silu(z) * bf16(w * bf16(y * rn)). 16 lanes per
+// kernel, split or fused (prefill_gate_apart): out[t, hv, :] = silu(z) * bf16(w * bf16(y * rn)). 16 lanes per
 // (token, value head), lane j rows 8j..8j+7; the sum of y^2 runs in the order
 // of the chunk kernel's own epilogue (per 4 rows, then per 16, then over the
 // 8 groups of 16 pairwise), so that both paths give the same bits.
@@ -1365,13 +1363,10 @@ static int forced_chunk_waves() {
 // against apart, us: 16/32 heads six prompts of 1,000 tokens 179 / 176, four of
 // 512 92 / 86 (as split), eight of 2,048 (256 groups, in the kernel) 387 / 400;
 // 4/16 heads eight of 1 to 3,000 tokens 365 / 255.
-constexpr int kGateApartGroups = 256;
-namespace {
-bool gate_apart(int R, int Hk, int nseq, int waves) {
+bool prefill_gate_apart(int R, int Hk, int nseq, int waves, int cus) {
   if (waves < 8) return true;
-  return forced_chunk_waves() == 0 && (int64_t)nseq * Hk * R < kGateApartGroups;
+  return forced_chunk_waves() == 0 && (int64_t)nseq * Hk * R < cus;
 }
-}  // namespace
 
 int prefill_chunk_waves(int R, int Hk, int nseq, int total_tokens) {
   if (const int f = forced_chunk_waves()) return total_tokens > 0 ? f : 8;
@@ -1406,10 +1401,10 @@ size_t prefill_workspace_bytes(int R, int Hk, int total_tokens, int nseq, int wa
   return carve(nullptr, R, Hk, total_tokens, nseq, waves, y_scratch, nullptr);
 }
 
-size_t prefill_workspace_reserve_bytes(int R, int Hk, int max_tokens) {
-  // the largest call the split path takes: every sequence count it picks,
+size_t prefill_workspace_reserve_bytes(int R, int Hk, int max_tokens, int cus) {
+  // the largest call of each path: every sequence count the split path picks,
   // the gated epilogue's y scratch included
-  size_t most = prefill_workspace_bytes(R, Hk, max_tokens, 1, 8, true);
+  size_t most = prefill_workspace_bytes(R, Hk, max_tokens, 1, 8, prefill_gate_apart(R, Hk, 1, 8, cus));
   // a forced split takes any call: up to one sequence per token
   const int f = forced_chunk_waves();
   if (f == 2 || f == 4)
@@ -1477,7 +1472,7 @@ static hipError_t launch_split(const PrefillArgs& a, const Workspace& ws) {
                      0, a.total_tokens, ws.qn, ws.kn, ws.vc, ws.lg, ws.beta, ws.rec, yb, nullptr,
                      a.xstride, nullptr, 0.0f, nullptr, a.status);
   e = hipGetLastError();
-  if (e != hipSuccess || !a.out) return e;
+  if (e != hipSuccess || !a.apart) return e;
   return launch_norm_gate(a, yb);
 }
 
@@ -1556,7 +1551,7 @@ static hipError_t launch_split_pipelined(const PrefillArgs& a, const Workspace& 
   hipError_t j = hipEventRecord(ev[1 + segs], a.aux);
   if (j == hipSuccess) j = hipStreamWaitEvent(a.stream, ev[1 + segs], 0);
   if (e == hipSuccess) e = j;
-  if (e != hipSuccess || !a.out) return e;
+  if (e != hipSuccess || !a.apart) return e;
   return launch_norm_gate(a, yb);
 }
 
@@ -1565,7 +1560,7 @@ static hipError_t launch_prefill_r(const PrefillArgs& a) {
   const int Hv = a.Hk * R;
   const int D = 2 * a.Hk * kDk + Hv * kDv;
   Workspace ws;
-  carve(a.workspace, R, a.Hk, a.total_tokens, a.nseq, a.waves, a.out && !a.y, &ws);
+  carve(a.workspace, R, a.Hk, a.total_tokens, a.nseq, a.waves, a.apart && !a.y, &ws);
   const int segs = a.aux && a.events ? a.segments : 1;
   if (segs > 1) {
     if (a.waves == 2) return launch_split_pipelined<R, 2>(a, ws, segs);
@@ -1588,9 +1583,8 @@ static hipError_t launch_prefill_r(const PrefillArgs& a) {
   if (a.waves == 2) return launch_split<R, 2>(a, ws);
   if (a.waves == 4) return launch_split<R, 4>(a, ws);
   const int units = Hv * a.nseq;
-  const bool apart = a.out && a.total_tokens > 0 && gate_apart(R, a.Hk, a.nseq, a.waves);
-  uint16_t* yb = apart && !a.y ? ws.y : a.y;
-  if (a.out && !apart)
+  uint16_t* yb = a.apart && !a.y ? ws.y : a.y;
+  if (a.out && !a.apart)
     hipLaunchKernelGGL((prefill_chunk_kernel<R, true, 8>), dim3(units), dim3(512), 0, a.stream,
                        a.state, a.slot_ids, a.cu_seqlens, a.num_slots, a.Hk, a.total_tokens, 0,
                        a.total_tokens, ws.qn, ws.kn, ws.vc, ws.lg, ws.beta, nullptr, a.y,
@@ -1600,7 +1594,7 @@ static hipError_t launch_prefill_r(const PrefillArgs& a) {
                        a.state, a.slot_ids, a.cu_seqlens, a.num_slots, a.Hk, a.total_tokens, 0,
                        a.total_tokens, ws.qn, ws.kn, ws.vc, ws.lg, ws.beta, nullptr, yb, nullptr,
                        a.xstride, nullptr, 0.0f, nullptr, a.status);
-  if ((e = hipGetLastError()) != hipSuccess || !apart) return e;
+  if ((e = hipGetLastError()) != hipSuccess || !a.apart) return e;
   return launch_norm_gate(a, yb);
 }
 

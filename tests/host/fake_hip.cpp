@@ -23,7 +23,9 @@ bool fail_embed = false;  // set by the test: embedding launches fail
 bool capture = false;     // set by the test: stream capture records the stand-in launches
 bool split = false;       // set by the test: prefill calls take the split path (2-wave groups)
 gdn::AttnArgs attn;       // of the last attention launch
+gdn::PrefillArgs prefill; // of the last prefill launch
 size_t malloc_bytes = 0;  // size of the last hipMalloc
+size_t malloc_limit = ~(size_t)0;  // set by the test: larger ones fail
 int graphs_live = 0, graphs_destroyed = 0, graphs_made = 0;
 std::vector<std::function<void()>>* recording = nullptr;  // the capture in progress
 }
@@ -32,6 +34,7 @@ extern "C" {
 
 hipError_t hipMalloc(void** ptr, size_t size) {
   gdn_fake::malloc_bytes = size;
+  if (size > gdn_fake::malloc_limit) return hipErrorOutOfMemory;
   *ptr = std::calloc(1, size ? size : 1);
   return *ptr ? hipSuccess : hipErrorOutOfMemory;
 }
@@ -170,13 +173,17 @@ int prefill_pipeline_segments(int waves, int nseq, int total_tokens, int groups,
              ? std::min(8, total_tokens / 4096)
              : 1;
 }
+bool prefill_gate_apart(int R, int Hk, int nseq, int waves, int cus) {
+  return waves < 8 || nseq * Hk * R < cus;
+}
 size_t prefill_workspace_bytes(int R, int Hk, int T, int nseq, int waves, bool y_scratch) {
   const size_t Hv = (size_t)Hk * R;
   size_t b = (size_t)T * (2 * (size_t)Hk * kDk * 2 + Hv * kDv * 2 + Hv * 6) + 5 * 256;
-  if (waves < 8) b += (size_t)(T / 64 + nseq) * Hv * 17408 + (y_scratch ? (size_t)T * Hv * kDv * 2 : 0);
+  if (waves < 8) b += (size_t)(T / 64 + nseq) * Hv * 17408;
+  if (y_scratch) b += (size_t)T * Hv * kDv * 2;
   return b;
 }
-size_t prefill_workspace_reserve_bytes(int R, int Hk, int T) {
+size_t prefill_workspace_reserve_bytes(int R, int Hk, int T, int) {
   return prefill_workspace_bytes(R, Hk, T, 1, 2, true);
 }
 static unsigned char g_scratch[(size_t)16 << 20];
@@ -185,7 +192,13 @@ hipError_t noalloc_scratch(void** out) {
   *out = g_scratch;
   return hipSuccess;
 }
-hipError_t launch_prefill(const PrefillArgs&) { return hipSuccess; }
+hipError_t launch_prefill(const PrefillArgs& a) {
+  gdn_fake::prefill = a;
+  return a.workspace_bytes < prefill_workspace_bytes(a.R, a.Hk, a.total_tokens, a.nseq, a.waves,
+                                                     a.apart && !a.y)
+             ? hipErrorInvalidValue
+             : hipSuccess;
+}
 size_t attn_workspace_bytes(int T, int Hq, int64_t chunks) {
   return (size_t)T * Hq * 256 * 2 + (size_t)chunks * 16 * 260 * 4 + 256;
 }

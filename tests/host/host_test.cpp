@@ -9,6 +9,8 @@
 #include <cstring>
 #include <vector>
 
+#include <hip/hip_runtime_api.h>
+
 #include "gdn.h"
 #include "gdn_common.h"
 
@@ -17,7 +19,9 @@ extern bool fail_embed;  // fake_hip.cpp: the next embedding launches fail
 extern bool capture;     // fake_hip.cpp: stream capture makes (empty) graphs
 extern bool split;       // fake_hip.cpp: prefill calls take the split path
 extern gdn::AttnArgs attn;  // fake_hip.cpp: arguments of the last attention launch
+extern gdn::PrefillArgs prefill;  // fake_hip.cpp: arguments of the last prefill launch
 extern size_t malloc_bytes;  // fake_hip.cpp: size of the last device allocation
+extern size_t malloc_limit;  // fake_hip.cpp: larger device allocations fail
 extern int graphs_live, graphs_destroyed, graphs_made;
 }
 
@@ -173,6 +177,60 @@ static int test_pool() {
   gdn_fake::split = false;
   uint32_t flags = 1;
   CHECK(gdn_pool_check(pool, nullptr, &flags) == GDN_OK && flags == 0);
+  CHECK(gdn_pool_destroy(pool) == GDN_OK);
+  return 0;
+}
+
+// Under capture, and when the device has no memory left, a prefill call whose
+// schedule wants more workspace than the pool holds takes the fused schedule
+// with the epilogue in its kernel instead of growing the buffer or failing.
+static int test_prefill_workspace_limits() {
+  gdn_pool_desc d{1, 8, 16, 32, 128, 128, 4, 0};
+  gdn_pool* pool = nullptr;
+  CHECK(gdn_pool_create(&d, &pool) == GDN_OK);
+  std::vector<std::vector<char>> keep;
+  const int D = 8192, V = 4096, T = 1024;
+  int32_t* ids = dev_alloc<int32_t>(keep, 4);
+  for (int i = 0; i < 4; ++i) ids[i] = i;
+  int32_t* cu = dev_alloc<int32_t>(keep, 5);
+  for (int i = 0; i < 5; ++i) cu[i] = i * T / 4;
+  uint16_t* x = dev_alloc<uint16_t>(keep, (size_t)2 * T * (D + V));
+  uint16_t* ab = dev_alloc<uint16_t>(keep, (size_t)2 * T * 64);
+  float* al = dev_alloc<float>(keep, 32);
+  float* dt = dev_alloc<float>(keep, 32);
+  uint16_t* cw = dev_alloc<uint16_t>(keep, (size_t)D * 4);
+  uint16_t* nw = dev_alloc<uint16_t>(keep, 128);
+  uint16_t* y = dev_alloc<uint16_t>(keep, (size_t)2 * T * V);
+  auto plain = [&](int tokens) {
+    cu[4] = tokens;
+    return gdn_prefill_varlen(pool, 0, ids, cu, 4, tokens, x, ab, al, dt, cw, y, nullptr);
+  };
+  auto gated = [&](int tokens) {
+    cu[4] = tokens;
+    return gdn_prefill_varlen_gated(pool, 0, ids, cu, 4, tokens, x, D + V, ab, 64, al, dt, cw, nw,
+                                    1e-6f, y, nullptr, nullptr);
+  };
+  CHECK(plain(T) == GDN_OK && gdn_fake::prefill.waves == 8);
+  void* const held = gdn_fake::prefill.workspace;
+  gdn_fake::capture = true;
+  CHECK(hipStreamBeginCapture(nullptr, hipStreamCaptureModeGlobal) == hipSuccess);
+  CHECK(gated(T) == GDN_OK && gdn_fake::prefill.waves == 8 && !gdn_fake::prefill.apart);
+  gdn_fake::split = true;
+  CHECK(plain(T) == GDN_OK && gdn_fake::prefill.waves == 8);
+  CHECK(gated(T) == GDN_OK && gdn_fake::prefill.waves == 8 && !gdn_fake::prefill.apart);
+  CHECK(gdn_fake::prefill.workspace == held);
+  hipGraph_t graph = nullptr;
+  CHECK(hipStreamEndCapture(nullptr, &graph) == hipSuccess && hipGraphDestroy(graph) == hipSuccess);
+  gdn_fake::capture = false;
+  // outside a capture the buffer grows and the schedule is the library's
+  CHECK(gated(T) == GDN_OK && gdn_fake::prefill.waves == 2 && gdn_fake::prefill.apart);
+  gdn_fake::malloc_limit = gdn::prefill_workspace_bytes(2, 16, 2 * T, 4, 8, false);
+  CHECK(gated(2 * T) == GDN_OK && gdn_fake::prefill.waves == 8 && !gdn_fake::prefill.apart);
+  gdn_fake::malloc_limit = 1 << 20;
+  CHECK(gdn_pool_reserve(pool, 8 * T, nullptr) == GDN_ERR_OOM);
+  gdn_fake::malloc_limit = ~(size_t)0;
+  CHECK(plain(2 * T) == GDN_OK && gdn_fake::prefill.waves == 2);
+  gdn_fake::split = false;
   CHECK(gdn_pool_destroy(pool) == GDN_OK);
   return 0;
 }
@@ -432,7 +490,7 @@ static int test_exec_graphs_follow_pool_buffer() {
 }
 
 int main() {
-  if (test_qlinear_plan() || test_pool() || test_kv() || test_kv_max_workers() || test_exec() ||
+  if (test_qlinear_plan() || test_pool() || test_prefill_workspace_limits() || test_kv() || test_kv_max_workers() || test_exec() ||
       test_exec_graphs_follow_pool_buffer())
     return 1;
   std::printf("ALL OK (%d checks)\n", g_checks);

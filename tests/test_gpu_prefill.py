@@ -465,6 +465,56 @@ def test_prefill_gated_bad_slot_leaves_its_rows(gpu, Hk, Hv, lens):
     assert np.array_equal(res[0][cu[1]:], res[1][cu[1]:])
 
 
+def test_prefill_captured_on_a_workspace_of_another_schedule(gpu):
+    """A pool whose workspace an eight-prompt call (fused schedule) has sized,
+    then calls of the same token count whose own schedule wants more (four
+    prompts, split; gated) captured in a graph: the capture succeeds, and
+    replays equal eager calls on another pool, bit for bit."""
+    import gdn_amd
+    import torch
+    say("gdn_prefill_varlen_gated captured", "8 x 512, then 4 x 1024")
+    rng = np.random.default_rng(665)
+    Hk, Hv, T = 16, 32, 4096
+    D = conv_dim(Hk, Hv)
+    p = gen_layer_params(rng, Hk, Hv)
+    mixed, ab = gen_tokens(rng, T, Hk, Hv)
+    qkvz = np.concatenate([mixed, gen_tokens(rng, T, Hk, Hv)[0][:, :Hv * DV]], axis=1)
+    md, qd = dev(mixed), dev(qkvz)
+    args = (dev(ab), dev(p["A_log"]), dev(p["dt_bias"]), dev(p["conv_w"]))
+    norm_w = dev(O.f32_to_bf16(np.ones(DV, np.float32)))
+    ids8, ids4 = _ids(np.arange(8, dtype=np.int32)), _ids(np.arange(4, dtype=np.int32))
+    cu8, cu4 = (dev(np.arange(0, T + 1, T // n).astype(np.int32)) for n in (8, 4))
+    pools = [gdn_amd.Pool(1, 8, Hk, Hv) for _ in range(2)]
+    outs = [torch.zeros((T, Hv, DV), dtype=torch.int16, device=gpu) for _ in range(4)]
+
+    def calls(pool, y, out):
+        pool.prefill(0, ids4, cu4, T, md, *args, y)
+        pool.prefill_gated(0, ids4, cu4, T, qd, *args, norm_w, 1e-6, out)
+
+    for pool in pools:
+        pool.prefill(0, ids8, cu8, T, md, *args, outs[0])
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(stream):
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=stream):
+            calls(pools[1], outs[2], outs[3])
+    torch.cuda.synchronize()
+    for step in range(3):
+        calls(pools[0], outs[0], outs[1])
+        graph.replay()
+        junk = torch.randn(1 << 20, device=gpu).sum()
+        torch.cuda.synchronize()
+        assert torch.isfinite(junk)
+        assert torch.equal(outs[0], outs[2]) and torch.equal(outs[1], outs[3]), step
+        for a, b in zip(*(_read(pool, 0, np.arange(8, dtype=np.int32), gpu) for pool in pools)):
+            assert np.array_equal(a, b), step
+    for pool in pools:
+        assert pool.check() == 0
+        pool.close()
+
+
 def test_prefill_one_long_prompt_pipelined_matches_one_pass(gpu, prefill_segments):
     """One 16,384-token prompt takes the split path in 4 segments by default;
     its y, state and conv window equal the one-pass call's bit for bit, and a
