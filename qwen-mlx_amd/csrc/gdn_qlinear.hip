@@ -885,6 +885,22 @@ hipError_t launch_qlinear_pack(const QLinearPackArgs& a) {
 hipError_t launch_qlinear(const QLinearArgs& a) {
   if (a.defer) *a.defer = QPartial{};
   const QLinearPlan plan = qlinear_plan(a.K, a.Npad, a.M, a.part_tiles);
+  // The kernels reach a call's rows (decode) or four rows of a copy (tiles) by
+  // 32-bit byte offsets; rows further apart than that go one by one.
+  const int reach = plan.kind == QLinearPlan::kDecode ? a.M : a.M < 4 ? a.M : 4;
+  if (reach > 1 && a.xs > (UINT32_MAX / 2 - a.K) / (reach - 1)) {
+    QLinearArgs c = a;
+    c.M = 1;
+    c.defer = nullptr;
+    c.xsplit = nullptr;
+    for (int m = 0; m < a.M; ++m) {
+      c.x = a.x + m * a.xs;
+      c.y = a.y + m * a.ys;
+      hipError_t e = launch_qlinear(c);
+      if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+  }
   if (plan.kind == QLinearPlan::kWide) {
     const bool xs = a.xsplit != nullptr;
     if (a.K > 2048) return xs ? launch_tile<4, 16, 1>(a) : launch_tile<4, 16, 0>(a);

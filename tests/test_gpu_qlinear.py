@@ -234,6 +234,34 @@ def test_qlinear_tiles_and_slices_sampled(gpu, M, K, N):
     layer.close()
 
 
+@pytest.mark.parametrize("M,xs", [(2, (1 << 31) - 520), (2, 1 << 31), (66, 715_827_888)])
+def test_qlinear_rows_far_apart(gpu, M, xs):
+    """x rows whose byte offsets pass 32 bits: within the rows of a decode
+    call, and (66 rows, 93 GB apart) within the four rows of a tile's copy."""
+    import torch
+    K, rows = 512, [80]
+    say("gdn_qlinear_forward", f"M={M} xs={xs}")
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 2.5 * M * xs:
+        pytest.skip("needs more free device memory")
+    rng = np.random.default_rng(509)
+    parts = _parts(rng, K, rows)
+    x = O.f32_to_bf16(rng.standard_normal((M, K)).astype(np.float32))
+    buf = torch.empty((M - 1) * xs + K, dtype=torch.int16, device=gpu)
+    xd = torch.as_strided(buf, (M, K), (xs, 1))
+    xd.copy_(dev(x))
+    layer = _layer(K, parts)
+    y = torch.full((M, 84), -1, dtype=torch.int16, device=gpu)
+    layer.forward(xd, y)
+    torch.cuda.synchronize()
+    assert bool((y[:, 80:] == -1).all())
+    yr, ye, mag = O.qmatmul_w4(x, *_merged(parts))
+    _check(host(y)[:, :80], ye, mag, yr, f"qlinear rows {xs} apart")
+    layer.close()
+    del buf, xd
+    torch.cuda.empty_cache()
+
+
 def test_qlinear_output_feeds_gated_decode_in_place(gpu):
     """Hidden states -> merged q|k|v|z|b|a projection -> gdn_decode_gated reading
     qkvz and ab as column slices of the one output (no copies), against the
