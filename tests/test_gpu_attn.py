@@ -270,7 +270,7 @@ def test_attention_tiles_equal_chunks(gpu, Hq, Hkv):
 
 
 def test_attention_long_context_splits(gpu):
-    """A 2,500-token context (three 1,024-key splits) built by prefill steps of
+    """A 2,500-token context (seven 384-key chunks) built by prefill steps of
     1,000 and 1,500 tokens, then two decode steps, against the oracle."""
     import gdn_amd
     say("gdn_attn_forward", "long context, 3 splits")
@@ -289,6 +289,73 @@ def test_attention_long_context_splits(gpu):
         _run_step(kv, seqs, [1], [1], gpu, label=f"decode at {kv.length(1)} keys")
     assert kv.length(1) == 2502
     kv.close()
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(16, 2), (16, 4)])
+def test_attention_combine_many_chunks(gpu, Hq, Hkv):
+    """Contexts on either side of 32 chunks of 384 keys (the combine kernel's
+    form of one dimension per lane) and of 64 (its reload), with scores spread
+    enough that a token's running maximum moves from chunk to chunk. Decode
+    tokens against the oracle, a short sequence in the same step against the
+    same step without the long one, and a 1,000-token prompt behind 24,577 keys
+    on tiles against the same tokens in two steps on chunks, bit for bit."""
+    import torch
+
+    import gdn_amd
+    say("gdn_attn_forward", f"many chunks Hq={Hq} Hkv={Hkv}")
+    rng = np.random.default_rng(1440 + Hkv)
+    ka, kb = (gdn_amd.KVCache(1, 2, 406, 404, Hq, Hkv, max_step_tokens=8192) for _ in range(2))
+    seqs = _Seqs(rng, Hq, Hkv, 1)
+    seqs.w = [tuple(O.f32_to_bf16(2 * O.bf16_to_f32(w)) for w in seqs.w[0])]  # score deviation 4
+    w = (dev(seqs.w[0][0]), dev(seqs.w[0][1]))
+    gen = torch.Generator(device=gpu)
+    gen.manual_seed(1440)
+
+    def rows(n):
+        return [torch.randn((n, c), device=gpu, generator=gen).bfloat16().view(torch.int16)
+                for c in (Hq * 2 * HD, Hkv * HD, Hkv * HD)]
+
+    def forward(kv, slots, ntok, q, k, v):
+        out = torch.empty((sum(ntok), Hq * HD), dtype=torch.int16, device=gpu)
+        kv.step(slots, ntok)
+        kv.forward(0, q, k, v, *w, EPS, THETA, ROT, out)
+        return out
+
+    def extend(to):  # both caches' long sequence, by the same prompt steps
+        while (n := min(to - ka.length(1), 8192)) > 0:
+            r = rows(n)
+            assert torch.equal(forward(ka, [1], [n], *r), forward(kb, [1], [n], *r))
+
+    short = rows(40)
+    for kv in (ka, kb):
+        forward(kv, [0], [40], *short)
+    for keys in (12287, 24575):
+        extend(keys)
+        for _ in range(2):  # a decode token makes 32 (64) chunks, the next 33 (65)
+            for s in (0, 1):
+                seqs.cache[(0, s)] = tuple(host(a) for a in ka.read(0, s))
+            q, k, v = seqs.rows(2)
+            qd, kd, vd = dev(q), dev(k), dev(v)
+            both = forward(ka, [1, 0], [1, 1], qd, kd, vd)
+            alone = [forward(kb, [s], [1], qd[i:i + 1], kd[i:i + 1], vd[i:i + 1])
+                     for i, s in enumerate((1, 0))]
+            assert torch.equal(both, torch.cat(alone))
+            for i, s in enumerate((1, 0)):
+                ref = O.bf16_to_f32(seqs.oracle(0, s, q[i:i + 1], k[i:i + 1], v[i:i + 1]))
+                err = rel_l2(O.bf16_to_f32(host(both[i:i + 1])), ref)
+                say("many chunks", f"slot {s} at {ka.length(s)} keys: relL2 {err:.2e}")
+                assert err <= 1e-2
+    n, tpt = 1000, 128 * Hkv // Hq
+    nb = [-(-(ka.length(1) + min(k + tpt, n)) // 32) for k in range(0, n, tpt)]
+    assert sum(nb) * Hkv > 100 * max(nb), "the step would not take the tile route"
+    assert sum(nb[:(500 + tpt - 1) // tpt]) * Hkv < 100 * nb[0], "half of it would"
+    q, k, v = rows(n)
+    whole = forward(ka, [1], [n], q, k, v)
+    halves = [forward(kb, [1], [500], *(a[i:i + 500] for a in (q, k, v))) for i in (0, 500)]
+    torch.cuda.synchronize()
+    assert torch.equal(whole, torch.cat(halves))
+    ka.close()
+    kb.close()
 
 
 @pytest.mark.parametrize("workers", [1, 3])
