@@ -576,7 +576,8 @@ static gdn_status prefill_common(gdn_pool* pool, int32_t layer, const int32_t* s
   // (where the pool's buffer cannot grow), and when the device has no memory left.
   const int R = pool->R, Hk = pool->d.num_k_heads;
   int waves = gdn::prefill_chunk_waves(R, Hk, nseq, total_tokens);
-  bool apart = out && total_tokens > 0 && gdn::prefill_gate_apart(R, Hk, nseq, waves, pool->cus);
+  bool apart = out && total_tokens > 0 &&
+               gdn::prefill_gate_apart(R, Hk, nseq, total_tokens, waves, pool->cus);
   size_t need = gdn::prefill_workspace_bytes(R, Hk, total_tokens, nseq, waves, apart && !y);
   const size_t least = gdn::prefill_workspace_bytes(R, Hk, total_tokens, nseq, 8, false);
   auto smallest = [&] {

@@ -346,7 +346,7 @@ int prefill_chunk_waves(int R, int Hk, int nseq, int total_tokens);
 // chunk kernel has `groups` work-groups, on a device of `cus` CUs (1: one
 // pass, no second stream).
 int prefill_pipeline_segments(int waves, int nseq, int total_tokens, int groups, int cus);
-bool prefill_gate_apart(int R, int Hk, int nseq, int waves, int cus);
+bool prefill_gate_apart(int R, int Hk, int nseq, int total_tokens, int waves, int cus);
 // y_scratch: the epilogue runs apart and the caller brings no y.
 size_t prefill_workspace_bytes(int R, int Hk, int total_tokens, int nseq, int waves, bool y_scratch);
 size_t prefill_workspace_reserve_bytes(int R, int Hk, int max_tokens, int cus);

@@ -1358,13 +1358,20 @@ static int forced_chunk_waves() {
 // over y (prefill_norm_gate_kernel): always on the split path, and on the fused
 // one while the chunk kernel's groups are fewer than the CUs. There the chunk
 // kernel is bound by the chain of its longest prompt, to which the epilogue in
-// the kernel adds about 2.6 us per chunk; a pass over y, z and out costs 9.6 ns
-// per chunk and sequence-head. Per gated call, epilogue in the chunk kernel
-// against apart, us: 16/32 heads six prompts of 1,000 tokens 179 / 176, four of
-// 512 92 / 86 (as split), eight of 2,048 (256 groups, in the kernel) 387 / 400;
-// 4/16 heads eight of 1 to 3,000 tokens 365 / 255.
-bool prefill_gate_apart(int R, int Hk, int nseq, int waves, int cus) {
+// the kernel adds about 2.6 us per chunk; the launch costs 2 us and a pass over
+// y, z and out 9.6 ns per chunk and sequence-head. Per gated call, epilogue in
+// the chunk kernel against apart, us: 16/32 heads six prompts of 1,000 tokens
+// 182 / 176, four of 512 92 / 86 (as split), eight of 2,048 (256 groups, in the
+// kernel) 387 / 400; 4/16 heads eight of 1 to 3,000 tokens 365 / 255.
+// Short calls do not pay the launch back: 16/32 heads, one prompt of 16 tokens
+// 19.0 / 20.9, of 48 20.8 / 21.4, of 64 22.1 / 22.0, of 128 30.0 / 27.0; six of 32
+// 23.0 / 25.4; seven of 16 22.5 / 24.7. The host knows the prompts' average, not
+// their lengths, and the two cost about as much where it errs: seven of 64 29.6 /
+// 32.9, but six of 8 and one of 400 70 / 59.
+constexpr int kGateShortTokens = 256, kGateShortAverage = 48;
+bool prefill_gate_apart(int R, int Hk, int nseq, int total_tokens, int waves, int cus) {
   if (waves < 8) return true;
+  if (total_tokens <= kGateShortTokens && total_tokens <= kGateShortAverage * nseq) return false;
   return forced_chunk_waves() == 0 && (int64_t)nseq * Hk * R < cus;
 }
 
@@ -1404,7 +1411,7 @@ size_t prefill_workspace_bytes(int R, int Hk, int total_tokens, int nseq, int wa
 size_t prefill_workspace_reserve_bytes(int R, int Hk, int max_tokens, int cus) {
   // the largest call of each path: every sequence count the split path picks,
   // the gated epilogue's y scratch included
-  size_t most = prefill_workspace_bytes(R, Hk, max_tokens, 1, 8, prefill_gate_apart(R, Hk, 1, 8, cus));
+  size_t most = prefill_workspace_bytes(R, Hk, max_tokens, 1, 8, prefill_gate_apart(R, Hk, 1, kSplitMaxTokens, 8, cus));
   // a forced split takes any call: up to one sequence per token
   const int f = forced_chunk_waves();
   if (f == 2 || f == 4)

@@ -173,7 +173,7 @@ int prefill_pipeline_segments(int waves, int nseq, int total_tokens, int groups,
              ? std::min(8, total_tokens / 4096)
              : 1;
 }
-bool prefill_gate_apart(int R, int Hk, int nseq, int waves, int cus) {
+bool prefill_gate_apart(int R, int Hk, int nseq, int, int waves, int cus) {
   return waves < 8 || nseq * Hk * R < cus;
 }
 size_t prefill_workspace_bytes(int R, int Hk, int T, int nseq, int waves, bool y_scratch) {

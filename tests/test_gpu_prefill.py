@@ -392,6 +392,10 @@ def test_prefill_pipelined_segments_match_one_pass(gpu, prefill_waves, prefill_s
     (16, 32, [300, 1, 700, 900, 64]),     # 160 sequence-heads: fused
     (4, 16, [1024, 3, 700, 129, 512, 64, 40, 3700]),  # 128 sequence-heads, average 771
     (4, 4, [5000, 1, 3500]),              # 8,192 tokens and few groups, but not one prompt
+    (16, 32, [100, 3, 64, 1, 80, 8]),     # 256 tokens, 42 on average: epilogue in the kernel
+    (16, 32, [100, 3, 64, 1, 80, 9]),     # and one more: apart
+    (4, 16, [48]),                        # one short prompt: in the kernel
+    (4, 16, [49]),                        # apart
 ])
 def test_prefill_schedule_rule_edges_match_fused(gpu, prefill_waves, Hk, Hv, lens):
     """The library's own choice of schedule at the edges of its rule against
@@ -436,10 +440,12 @@ def test_prefill_schedule_rule_edges_match_fused(gpu, prefill_waves, Hk, Hv, len
         assert np.array_equal(a, b), f"output {i} differs from the fused schedule"
 
 
-@pytest.mark.parametrize("Hk,Hv,lens", [(16, 32, [70, 200, 40]), (16, 32, [300, 600, 129])])
+@pytest.mark.parametrize("Hk,Hv,lens", [(16, 32, [70, 200, 40]), (16, 32, [300, 600, 129]),
+                                        (16, 32, [20, 70, 9])])
 def test_prefill_gated_bad_slot_leaves_its_rows(gpu, Hk, Hv, lens):
     """A sequence with a slot id out of range is skipped whole where the
-    epilogue is a kernel of its own (fused and split schedule): its rows of
+    epilogue is a kernel of its own (fused and split schedule) and where it is
+    in the chunk kernel (short calls): its rows of
     out keep what they held, the others' equal a call without it."""
     import gdn_amd
     import torch
