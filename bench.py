@@ -502,7 +502,13 @@ def qlinear_bench(args):
         roof = {"bound": "mfma", "achieved": round(tf, 2), "peak": PEAK_BF16_TFLOPS,
                 "unit": "TFLOP/s", "frac": round(tf / PEAK_BF16_TFLOPS, 4), "traffic": None,
                 "flop_per_launch": flops}
-    roof.update({"kernel": "qlinear_decode_kernel<8, 2>" if M <= 64 else "qlinear_kernel<2, 4, 2, 2>",
+    if M <= 64:
+        kernel = f"qlinear_decode_kernel<8, 2, {1 if M <= 16 else 2 if M <= 32 else 4}, false>"
+    elif -(-M // 64) * -(-N // 128) >= 2304:  # group sums formed up front
+        kernel = "qlinear_xsum_kernel + qlinear_tile_kernel<4, 8, 2>"
+    else:
+        kernel = "qlinear_tile_kernel<4, 8, 0>"
+    roof.update({"kernel": kernel,
                  "kernel_avg_us": round(avg_ms * 1e3, 2),
                  "kernel_timing": "HIP events around each step's back-to-back launches / launches"})
     out = {

@@ -271,8 +271,9 @@ gdn_status gdn_prefill_varlen_noalloc(gdn_pool* pool, int32_t layer, const int32
                                       uint16_t* y, void* stream);
 
 /* gdn_prefill_varlen on merged projection rows with the RMSNormGated epilogue
- * fused into the chunk kernel's readout (qwen3_5.rs:660-665 after the S>1
- * path): out [total_tokens, Hv, Dv] = silu(z) * rms_norm(y, norm_w, norm_eps)
+ * (qwen3_5.rs:660-665 after the S>1 path), in the chunk kernel's readout or as a
+ * kernel of its own over the ungated rows, by the call's
+ * size (the same bits): out [total_tokens, Hv, Dv] = silu(z) * rms_norm(y, norm_w, norm_eps)
  * per (token, value head). qkvz [total_tokens, row_stride] holds q|k|v in
  * columns [0, D) and z in [D, D + Hv*Dv) (row_stride >= D + Hv*Dv, a multiple
  * of 8, qkvz 16-byte aligned); ab [total_tokens, ab_stride] holds b|a in its

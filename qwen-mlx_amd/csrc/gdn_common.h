@@ -262,7 +262,7 @@ struct QLinearArgs {
 // larger calls go in pieces of this many rows.
 constexpr int kQLinearSumRows = 16384;
 // 64 x 128 f32 tiles (32 KiB each) of a layer's partial-sum workspace: a
-// K-sliced call on tiles is at most this many work-groups.
+// K-sliced call on tiles is at most this many work-groups, two per CU of 256.
 constexpr int kQLinearPartTiles = 512;
 // Calls of at least kQLinearSumTiles tiles (three rounds of the 768 work-groups
 // that fit 256 CUs) on layers of at least kQLinearSumColumns columns form the

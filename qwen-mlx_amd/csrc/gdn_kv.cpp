@@ -69,12 +69,16 @@ constexpr int kTileMinTokens = 16;
 
 // Tiles or chunks for the step's prompts: `work` 32-key blocks over all their
 // tiles, `longest` of the longest one. A tile block takes about 2.07 us on its CU
-// and a tile's blocks run one after the other; the chunk route takes about 19.5
-// ns per tile block with the whole chip at work on it (16/2 heads, measured on
-// 1,024 to 4,096 new tokens behind 0 to 4,096 cached ones). So tiles win once
-// their work passes 100 of the longest: 2,048 tokens 157 us against 185, behind
-// 2,048 cached ones 281 against 490, 4,096 tokens 322 against 710; 512 tokens
-// behind 4,096 stay on chunks, 145 against 304.
+// and a tile's blocks run one after the other; the chunk route takes 13 to 20 ns
+// per tile block with the whole chip (256 CUs) at work on it. So tiles win once
+// their work passes 100 to 150 of the longest, by shape; the line lies at the
+// lower end, where short prompts gain. Tiles against chunks, us, with work /
+// longest: 16/2 heads 32 prompts of 20 tokens 27.5 / 31.5 (128), eight of 300
+// 57 / 90 (160), 2,048 tokens 156 / 151 (130), behind 2,048 cached ones 282 / 388
+// (193), 4,096 tokens 320 / 553 (258); 8/2 four of 1,000 96 / 106 (132), 4,096
+// tokens 286 / 259 (129); 32/4 1,024 tokens 96 / 105 (132), 2,048 190 / 323 (260).
+// It errs most on a short prompt behind a long context: 16/2 1,024 tokens behind
+// 4,096 339 / 309 (116), 32/4 512 behind 4,096 312 / 232 (121).
 bool use_tiles(int64_t work, int64_t longest) { return work > 100 * longest; }
 
 int max_workers(const gdn_kv_desc& d) { return d.max_workers > 0 ? d.max_workers : kReuseWorkers; }

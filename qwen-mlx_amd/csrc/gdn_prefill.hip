@@ -29,7 +29,9 @@ constexpr int kTT = 64;  // tokens per qkv_kernel work-group
 // The split path is taken for calls of at most kSplitMaxGroups sequence-heads
 // and kSplitMaxTokens tokens (its records take 272 bytes per token and value
 // head) whose prompts hold at least kSplitMinTokens tokens on average, or
-// kSplitMinTokensFull above 96 sequence-heads (see prefill_chunk_waves).
+// kSplitMinTokensFull above 96 sequence-heads (see prefill_chunk_waves). What
+// decides is the longest prompt's chain, but the lengths are on the device: the
+// average bounds it from below. The limits on sequence-heads are for 256 CUs.
 constexpr int kSplitMinTokens = 256;
 constexpr int kSplitMinTokensFull = 768;
 constexpr int kSplitMaxGroups = 128;
@@ -1337,7 +1339,7 @@ __global__ __launch_bounds__(256) void prefill_norm_gate_kernel(
 // head)) where the fused kernel would leave at least half of the CUs idle: up
 // to 128 sequence-heads, one work-group each. A chunk then takes about 3.3 us
 // of the longest prompt's chain against 5.6, and the forming of the blocks is
-// paid up front. Measured per call, fused against split, us: 16/32 heads one
+// paid up front. Measured per call on 256 CUs, fused against split, us: 16/32 heads one
 // prompt of 128 tokens 23.7 / 23.9, 256 33.7 / 30.1, 512 55 / 46; three of 37,
 // 512 and 1,200 118 / 99; four of 512 71.4 / 73.3, of 128, 512, 1,000 and 2,048
 // 193 / 164, of 2,048 226 / 222, of 16,384 1,648 / 1,610; 4/16 heads six of
@@ -1387,7 +1389,8 @@ int prefill_chunk_waves(int R, int Hk, int nseq, int total_tokens) {
 // groups, one per CU, number at most half the CUs), a call of at least two
 // segments of kPipeSegmentTokens runs its qkv and form kernels one segment
 // ahead on a second stream, beside the chunk kernel of the previous segment.
-// Only one prompt is pipelined; several lose: segments cut the packed tokens, so a later prompt falls wholly into
+// Only one prompt is pipelined; several lose: segments cut the packed tokens,
+// so a later prompt falls wholly into
 // the last segments and its chain starts only after the first prompt's (two
 // 16,384-token prompts forced into segments: 1.72-1.75 ms per layer at 256
 // 2-wave groups, 1.68-1.72 at 128 4-wave groups, against 1.19 in one pass; at

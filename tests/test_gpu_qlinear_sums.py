@@ -18,7 +18,7 @@ Checks, in order:
   same bar for gdn_qlinear_forward on the same rows (the path that forms the
   sums itself).
 
-The same holds for the lm_head tiles (qlinear_tile_kernel<8, 1>, layers at
+The same holds for the lm_head tiles (qlinear_tile_kernel<MW, KT, 1>, layers at
 least 131,072 columns wide), checked on sampled columns of a 131,088-column
 layer at M = 1, 37 and 64.
 """
