@@ -45,7 +45,8 @@
  *     chunk records there, and gated calls may hold their ungated rows)
  *     synchronizes its stream and reallocates it, later
  *     calls at or below that size allocate nothing; gdn_pool_reserve sizes it
- *     for any call up to a token count. Under stream capture, and when the
+ *     for any call up to a token count (a graph that holds the buffer is not
+ *     replayed after it has moved). Under stream capture, and when the
  *     device has no memory left, such a call takes the schedule with the
  *     smallest workspace instead (16,576 bytes per token at 16 key / 32 value
  *     heads; the same bits) and grows the buffer only if that does not fit,
@@ -272,9 +273,9 @@ gdn_status gdn_prefill_varlen_noalloc(gdn_pool* pool, int32_t layer, const int32
 
 /* gdn_prefill_varlen on merged projection rows with the RMSNormGated epilogue
  * (qwen3_5.rs:660-665 after the S>1 path), in the chunk kernel's readout or as a
- * kernel of its own over the ungated rows, by the call's
- * size (the same bits): out [total_tokens, Hv, Dv] = silu(z) * rms_norm(y, norm_w, norm_eps)
- * per (token, value head). qkvz [total_tokens, row_stride] holds q|k|v in
+ * kernel of its own over the ungated rows, by the call's size (the same bits):
+ * out [total_tokens, Hv, Dv] = silu(z) * rms_norm(y, norm_w, norm_eps) per
+ * (token, value head). qkvz [total_tokens, row_stride] holds q|k|v in
  * columns [0, D) and z in [D, D + Hv*Dv) (row_stride >= D + Hv*Dv, a multiple
  * of 8, qkvz 16-byte aligned); ab [total_tokens, ab_stride] holds b|a in its
  * first 2*Hv columns. y [total_tokens, Hv, Dv] (the ungated output) may be

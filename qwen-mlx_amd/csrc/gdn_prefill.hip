@@ -68,8 +68,7 @@ size_t carve(void* base, int R, int Hk, int T, int nseq, int waves, bool y_scrat
   ws.rec = nullptr;
   ws.y = nullptr;
   if (waves < 8) ws.rec = static_cast<uint16_t*>(take((size_t)(T / 64 + nseq) * Hv * kRecStride));
-  if (y_scratch)
-    ws.y = static_cast<uint16_t*>(take((size_t)T * Hv * kDv * 2));
+  if (y_scratch) ws.y = static_cast<uint16_t*>(take((size_t)T * Hv * kDv * 2));
   if (w) *w = ws;
   return off;
 }
@@ -1294,10 +1293,10 @@ __global__ __launch_bounds__(512) void prefill_form_kernel(
 }
 
 // RMSNormGated epilogue (qwen3_5.rs:660-665) over y written by the ungated chunk
-// kernel, split or fused (prefill_gate_apart): out[t, hv, :] = silu(z) * bf16(w * bf16(y * rn)). 16 lanes per
-// (token, value head), lane j rows 8j..8j+7; the sum of y^2 runs in the order
-// of the chunk kernel's own epilogue (per 4 rows, then per 16, then over the
-// 8 groups of 16 pairwise), so that both paths give the same bits.
+// kernel, split or fused (prefill_gate_apart): out[t, hv, :] = silu(z) * bf16(w *
+// bf16(y * rn)). 16 lanes per (token, value head), lane j rows 8j..8j+7; the sum of
+// y^2 runs in the order of the chunk kernel's own epilogue (per 4 rows, then per
+// 16, then over the 8 groups of 16 pairwise), so that both paths give the same bits.
 __global__ __launch_bounds__(256) void prefill_norm_gate_kernel(
     const uint16_t* __restrict__ y, const uint16_t* __restrict__ zrow, int64_t xs,
     const uint16_t* __restrict__ norm_w, float norm_eps, uint16_t* __restrict__ out, int T, int Hv,
@@ -1389,12 +1388,11 @@ int prefill_chunk_waves(int R, int Hk, int nseq, int total_tokens) {
 // groups, one per CU, number at most half the CUs), a call of at least two
 // segments of kPipeSegmentTokens runs its qkv and form kernels one segment
 // ahead on a second stream, beside the chunk kernel of the previous segment.
-// Only one prompt is pipelined; several lose: segments cut the packed tokens,
-// so a later prompt falls wholly into
-// the last segments and its chain starts only after the first prompt's (two
-// 16,384-token prompts forced into segments: 1.72-1.75 ms per layer at 256
-// 2-wave groups, 1.68-1.72 at 128 4-wave groups, against 1.19 in one pass; at
-// 4/4 heads four of 16,384 2.46 ms against 0.92).
+// Only one prompt is pipelined; several lose: segments cut the packed tokens, so a
+// later prompt falls wholly into the last segments and its chain starts only after
+// the first prompt's (two 16,384-token prompts forced into segments: 1.72-1.75 ms
+// per layer at 256 2-wave groups, 1.68-1.72 at 128 4-wave groups, against 1.19 in
+// one pass; at 4/4 heads four of 16,384 2.46 ms against 0.92).
 // GDN_PREFILL_SEGMENTS = n forces n segments (1: one pass) on the split path.
 constexpr int kPipeSegmentTokens = 4096;
 
@@ -1414,7 +1412,8 @@ size_t prefill_workspace_bytes(int R, int Hk, int total_tokens, int nseq, int wa
 size_t prefill_workspace_reserve_bytes(int R, int Hk, int max_tokens, int cus) {
   // the largest call of each path: every sequence count the split path picks,
   // the gated epilogue's y scratch included
-  size_t most = prefill_workspace_bytes(R, Hk, max_tokens, 1, 8, prefill_gate_apart(R, Hk, 1, kSplitMaxTokens, 8, cus));
+  const bool apart = prefill_gate_apart(R, Hk, 1, kSplitMaxTokens, 8, cus);
+  size_t most = prefill_workspace_bytes(R, Hk, max_tokens, 1, 8, apart);
   // a forced split takes any call: up to one sequence per token
   const int f = forced_chunk_waves();
   if (f == 2 || f == 4)
